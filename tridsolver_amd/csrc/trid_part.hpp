@@ -745,39 +745,11 @@ struct CoefConst {
 // ORDER, VEC 0 only).  load() fills a, b, c of rows row0..row0+R-1 of the
 // system at element offset off (stride s) in arrays with the layout of
 // SysDesc array 0; rows past N are identity rows.
-//   CoefTransposed: the transposed system A^T of tridiag(A, B, C): sub-
-//                   diagonal c_{i-1}, diagonal b_i, super-diagonal a_{i+1}.
 //   CoefKappa:      the variable-diffusivity ADI operator along a line:
 //                   face values kf_{i+1/2} = (K_i + K_{i+1})/2 and, at rows
 //                   interior to the grid, a_i = -lam kf_{i-1/2},
 //                   c_i = -lam kf_{i+1/2}, b_i = 1 - a_i - c_i (identity rows
 //                   elsewhere); with transpose, its transposed operator.
-template <typename T>
-struct CoefTransposed {
-  static constexpr bool kArrays = false;
-  static constexpr bool kHook = true;
-  const T *__restrict__ A;
-  const T *__restrict__ B;
-  const T *__restrict__ C;
-  template <int R, typename I>
-  __device__ __forceinline__ void load(int row0, int N, bool, I off, I s,
-                                       T (&a)[R], T (&b)[R], T (&c)[R]) const {
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int row = row0 + r;
-      if (row < N) {
-        a[r] = row >= 1 ? ld_stream(at(C, off + (I)(row - 1) * s)) : T(0);
-        b[r] = ld_stream(at(B, off + (I)row * s));
-        c[r] = row + 1 < N ? ld_stream(at(A, off + (I)(row + 1) * s)) : T(0);
-      } else {
-        a[r] = T(0);
-        b[r] = T(1);
-        c[r] = T(0);
-      }
-    }
-  }
-};
-
 template <typename T>
 struct CoefKappa {
   static constexpr bool kArrays = false;
