@@ -44,8 +44,8 @@ EXTERN_C tridStatus_t tridAdiPlanDestroy(tridAdiPlan_t plan);
 /* Enqueues nsteps time steps; sync = 1 waits for them to finish.  From the
  * second consecutive call with the same arrays and nsteps >= 2 on, the steps
  * run as launches of a HIP graph of min(nsteps, 64) steps, captured at that
- * call (the plan keeps one such graph; the kernels are those of
- * tridAdiStage, so results are bitwise the same). */
+ * call (the plan keeps one such graph; it holds the same kernels, so results
+ * are bitwise the same). */
 EXTERN_C tridStatus_t tridAdiStep(tridAdiPlan_t plan, void *u, void *du,
                                   int nsteps, int sync);
 
@@ -53,7 +53,9 @@ EXTERN_C tridStatus_t tridAdiStep(tridAdiPlan_t plan, void *u, void *du,
  * 2 = y sweep, 3 = z sweep with u += , 4 = right-hand side fused with the x
  * sweep (for tests and per-kernel timing).  tridAdiStep uses 4, 2, 3 when
  * the plan supports the fused stage (tridAdiPlanDescribe says so) and u, du
- * are 16-byte aligned, else 0, 1, 2, 3. */
+ * are 16-byte aligned; else, and for some grids in place of stage 4, a kernel
+ * of its own for stages 0 and 1 together (lines of at most 834 points, arrays
+ * below 4 GiB, any alignment; "lines" in tridAdiPlanDescribe); else 0, 1, 2, 3. */
 EXTERN_C tridStatus_t tridAdiStage(tridAdiPlan_t plan, void *u, void *du,
                                    int stage);
 

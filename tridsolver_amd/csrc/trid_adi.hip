@@ -1,6 +1,7 @@
 // trid_adi.hip -- ADI heat-diffusion time stepping (include/trid_adi.h).
 //
-// One time step is four kernels on the library stream:
+// One time step is four kernels on the library stream (the first two fused
+// into one, k_adi_rhs_x or k_adi_rhs_xl, wherever the grid fits either):
 //   k_adi_rhs           du = lambda * (7-point Laplacian of u), 0 on the
 //                       boundary (apps/adi/src/preproc.cu:38-90 without the
 //                       nine coefficient arrays)
@@ -345,6 +346,172 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// Factors of the whole-line x sweep (k_adi_rhs_xl): the interior rows
+// 1 .. nx-2 of a line in chunks of R.  Every chunk but a shorter last one is
+// the same Toeplitz block, and the forward recurrence of the last one is a
+// prefix of it, so the per-row factors are one set for all lanes (kernel
+// arguments, i.e. scalar registers); what depends on the chunk -- the first
+// row's and the reduced system's factors, (6 + 3 levels) x ch values, value i
+// of chunk k at F[i * ch + k] -- is read per lane.
+template <typename T, int R>
+struct LineFactors {
+  T a, c;           // sub- and super-diagonal
+  T ri[R];          // 1 / pivot of row i >= 1
+  T ap[R], cp[R];   // row i after the forward sweep: y_i + ap y_0 + cp y_{i+1} = d
+  const T *F;
+};
+
+// The right-hand side + x sweep for lines of any length and arrays of any
+// element alignment: a wave takes lpw = 64 / ch whole lines of ch chunks each
+// (lanes past lpw * ch idle), i.e. one contiguous span, and its four
+// neighbour spans are the same span shifted by one line or one plane -- also
+// across the ends of a plane, where the shifted elements belong to no
+// interior point.  The 16-byte pieces (NP per lane cover the span) are loaded
+// at element alignment; piece indices off the array are clamped into it,
+// which touches pieces without interior points only.  R is odd, so that the
+// per-lane chunks, R elements apart in LDS, fall in distinct banks without
+// padding.  The host keeps nx >= 3 and the arrays below 4 GiB.
+// The separate right-hand side and x kernels it replaces were bound by their
+// launches, a second pass over du and per-lane row access; this one by its
+// loads (five spans per line) at 54-94 VGPRs, with about a third of the VALU
+// instructions of the in-kernel factors.  200 x 150 x 180 FP32: 33 -> 13 us
+// (70 -> 50 us per step); 201 x 150 x 177 FP64: 63 -> 22 (122 -> 81); 250^3
+// FP64 runs a step in 170 us, as fast as the fused kernel at 256^3.
+template <typename T, int R, int NP, int CP>
+__global__ void __launch_bounds__(256)
+    k_adi_rhs_xl(const T *__restrict__ u, T *__restrict__ du, unsigned n, int nx, int ny, int nz,
+                 T lam, LineFactors<T, R> lf, int ch, int lpw, int xcd) {
+  static_assert(R % 2 == 1 && R >= 3, "even chunk lengths have bank conflicts");
+  constexpr int E = Vec16<T>::n;
+  constexpr int SW = NP * kWave * E + (R + E) / E * E;  // chunk reads may run R past the span
+  using V = typename Vec16<T>::type;
+  typedef T VU __attribute__((ext_vector_type(E), aligned(sizeof(T))));
+  __shared__ __align__(16) T smem[4 * SW];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  unsigned blk = blockIdx.x;
+  if (xcd) {
+    const unsigned nb8 = gridDim.x & ~7u;
+    if (blk < nb8) blk = (blk & 7u) * (nb8 >> 3) + (blk >> 3);
+  }
+  const unsigned nlines = (unsigned)ny * (unsigned)nz;
+  const unsigned wl = (blk * 4 + (unsigned)wv) * (unsigned)lpw;  // the wave's first line
+  if (wl >= nlines) return;  // (no work-group barriers below)
+  const int nl = (int)(nlines - wl < (unsigned)lpw ? nlines - wl : (unsigned)lpw);
+  const unsigned p0 = wl * (unsigned)nx, nxy = (unsigned)nx * (unsigned)ny;
+  const int len = nl * nx;
+  T *buf = smem + wv * SW;
+  {
+    VU c[NP], ym[NP], yp[NP], zm[NP], zp[NP];
+    const unsigned top = n - E, elast = (unsigned)((len - 1) / E * E);
+    auto ld = [&](unsigned p) {
+      return *reinterpret_cast<const VU *>(at(u, p < top ? p : top));
+    };
+#pragma unroll
+    for (int v = 0; v < NP; v++) {
+      const unsigned e = (unsigned)(v * kWave + lane) * E;
+      const unsigned p = p0 + (e < elast ? e : elast);
+      c[v] = ld(p);
+      ym[v] = ld(p >= (unsigned)nx ? p - (unsigned)nx : 0u);
+      yp[v] = ld(p + (unsigned)nx);
+      zm[v] = ld(p >= nxy ? p - nxy : 0u);
+      zp[v] = ld(p + nxy);
+    }
+    // the stencil in the loaded layout, as k_adi_rhs_x; points off the
+    // interior get values nothing uses
+#pragma unroll
+    for (int v = 0; v < NP; v++) {
+      T left = lane_read(c[v][E - 1], lane > 0 ? lane - 1 : 0);
+      T right = lane_read(c[v][0], lane < kWave - 1 ? lane + 1 : kWave - 1);
+      const T prev_last = v > 0 ? lane_bcast(c[v > 0 ? v - 1 : 0][E - 1], kWave - 1) : T(0);
+      const T next_first = v + 1 < NP ? lane_bcast(c[v + 1 < NP ? v + 1 : 0][0], 0) : T(0);
+      if (lane == 0) left = prev_last;
+      if (lane == kWave - 1) right = next_first;
+      V sd;
+#pragma unroll
+      for (int t = 0; t < E; t++) {
+        const T l = t == 0 ? left : c[v][t > 0 ? t - 1 : 0];
+        const T r = t == E - 1 ? right : c[v][t + 1 < E ? t + 1 : 0];
+        sd[t] = rhs_point(l, r, ym[v][t], yp[v][t], zm[v][t], zp[v][t], c[v][t], lam);
+      }
+      *reinterpret_cast<V *>(buf + (v * kWave + lane) * E) = sd;
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+  const int ln = lane / ch, k = lane - ln * ch;
+  const bool on = ln < nl;
+  const int base = on ? ln * nx + 1 + k * R : 0;
+  const int m = nx - 2 - k * R;  // interior rows from the chunk's first on
+  const T *__restrict__ Fk = lf.F + k;
+  auto fv = [&](int i) { return Fk[i * ch]; };
+  T d[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) d[r] = buf[base + r];
+  // forward sweep; rows past the interior are identity rows with d = 0
+  {
+    T dp = m > 1 ? d[1] * lf.ri[1] : T(0);
+    d[1] = dp;
+#pragma unroll
+    for (int i = 2; i < R; i++) {
+      dp = m > i ? (d[i] - lf.a * dp) * lf.ri[i] : T(0);
+      d[i] = dp;
+    }
+  }
+  // the first row through the backward recurrence
+  T t = d[R - 2];
+#pragma unroll
+  for (int i = R - 3; i >= 1; i--) t = d[i] - lf.cp[i] * t;
+  const T fd = (d[0] - lf.c * t) * fv(0);
+  // reduced system over the line's chunks (consecutive lanes)
+  T fnd = lane_read(fd, k + 1 < ch ? lane + 1 : lane);
+  if (k + 1 >= ch) fnd = T(0);
+  T rd = (d[R - 1] - fv(3) * fd - fv(4) * fnd) * fv(5);
+  int j = 6;
+  for (int st = 1; st < ch; st <<= 1, j += 3) {
+    T md = lane_read(rd, k >= st ? lane - st : lane);
+    T pd = lane_read(rd, k + st < ch ? lane + st : lane);
+    if (k < st) md = T(0);
+    if (k + st >= ch) pd = T(0);
+    rd = (rd - fv(j) * md - fv(j + 1) * pd) * fv(j + 2);
+  }
+  T xm = lane_read(rd, k > 0 ? lane - 1 : lane);
+  if (k == 0) xm = T(0);
+  const T xf = fd - fv(1) * xm - fv(2) * rd;
+  // back substitution
+  T y[R];
+  y[0] = xf;
+  y[R - 1] = rd;
+#pragma unroll
+  for (int i = R - 2; i >= 1; i--)
+    y[i] = m > i ? d[i] - lf.ap[i] * xf - lf.cp[i] * y[i + 1] : T(0);
+  // the line's place: lines on the grid's faces keep du = 0
+  const unsigned line = wl + (unsigned)ln, kz = line / (unsigned)ny, jy = line - kz * (unsigned)ny;
+  const bool line_in = jy >= 1 && jy + 2 <= (unsigned)ny && kz >= 1 && kz + 2 <= (unsigned)nz;
+  __builtin_amdgcn_wave_barrier();
+  if (on) {
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      if (r < m) buf[base + r] = line_in ? y[r] : T(0);
+    if (k == 0) buf[base - 1] = T(0);
+    if (k == ch - 1) buf[base + m] = T(0);
+  }
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int v = 0; v < NP; v++) {
+    const int e = (v * kWave + lane) * E;
+    if (e + E <= len) {
+      const VU w = *reinterpret_cast<const V *>(buf + e);
+      VU *g = reinterpret_cast<VU *>(at(du, p0 + (unsigned)e));
+      if constexpr (CP == kCached) *g = w;
+      else __builtin_nontemporal_store(w, g);
+    } else {
+#pragma unroll
+      for (int q = 0; q < E; q++)
+        if (e + q < len) st_stream<CP>(at(du, p0 + (unsigned)(e + q)), buf[e + q]);
+    }
+  }
+}
+
 namespace {
 
 SysDesc grid_desc(int nx, int ny, int nz, int dir) {
@@ -373,6 +540,15 @@ SysDesc grid_desc(int nx, int ny, int nz, int dir) {
 
 using namespace tridhip;
 
+namespace {
+// Layout of the whole-line RHS + x kernel (k_adi_rhs_xl): chunk length,
+// chunks per line, lines per wave, 16-byte pieces per lane; R = 0 when the
+// grid does not fit the kernel.
+struct LinesLayout {
+  int R = 0, ch = 0, lpw = 0, np = 0;
+};
+}  // namespace
+
 struct tridAdiPlan_st {
   int nx = 0, ny = 0, nz = 0, dbl = 1, mode = 1;
   double lambda = 1.0;
@@ -384,6 +560,10 @@ struct tridAdiPlan_st {
   int fused_xcd = 0;        // XCD-contiguous block order of the fused kernel
   int fused_cc = 0;         // fused x sweep with precomputed factors
   void *fused_F[3] = {nullptr, nullptr, nullptr};  // their tables, chunk length 4, 8, 16
+  LinesLayout lines;        // R > 0: whole-line RHS + x sweep and its factors
+  double lines_f[3][16] = {};  // per-row factors ri, ap, cp
+  void *lines_F = nullptr;     // per-chunk factors (device)
+  int lines_first = 0;         // tridAdiStep prefers it to the fused kernel
   int cp = 0;               // cache policy of every stage's streaming accesses
   // y and z sweeps with precomputed factors (trid_cc.hpp): chunk length (0 =
   // the generic kernel), chunks per system and the factor table
@@ -484,6 +664,171 @@ hipError_t launch_fused(tridAdiPlan_st *p, T *u, T *du, hipStream_t st) {
   return hipGetLastError();
 }
 
+constexpr int kLinesRows[] = {5, 7, 9, 11, 13};
+
+LinesLayout lines_layout(int nx, int ny, int nz, size_t tsize) {
+  LinesLayout best;
+  const unsigned long long n = (unsigned long long)nx * ny * nz;
+  if (nx < 3 || n < 4 || n * tsize >= (1ULL << 32) || wide_index()) return best;
+  const int E = 16 / (int)tsize;
+  double cost = 0;
+  for (int R : kLinesRows) {
+    LinesLayout t;
+    t.R = R;
+    t.ch = (nx - 2 + R - 1) / R;
+    if (t.ch > kWave) continue;
+    t.lpw = kWave / t.ch;
+    // a span of short lines takes at most the pieces of its chunks' rows
+    const int np = (R + E - 1) / E;
+    t.lpw = std::min(t.lpw, np * kWave * E / nx);
+    if (t.lpw < 1) continue;
+    t.np = std::max(np - 1, (t.lpw * nx + kWave * E - 1) / (kWave * E));
+    // per line: loads and stencil of the pieces, the chunk sweeps, the rest
+    // (weights fitted to the step times of all five lengths on 14 grids)
+    const double c = (t.np * E * 10.0 + R * 8.0 + 60.0) / t.lpw;
+    if (!best.R || c < cost) {
+      best = t;
+      cost = c;
+    }
+  }
+  return best;
+}
+
+// Levels of the reduced system's PCR over ch chunks.
+int lines_levels(int ch) { return ilog2(ch); }
+
+// The factors of the whole-line x sweep: the recurrences of chunk_reduce,
+// eliminate_first and pcr_update on the coefficients, in double.  Per-row
+// factors to ri, ap, cp (R values each), per-chunk ones to F.
+template <typename T>
+void lines_factors(const CoefConst<T> &cf, int nx, const LinesLayout &L, double *ri, double *ap,
+                   double *cp, std::vector<T> &F) {
+  const double a = cf.a, b = cf.b, c = cf.c;
+  const int R = L.R, ch = L.ch;
+  ri[0] = ap[0] = cp[0] = 0;
+  for (int i = 1; i < R; i++) {
+    ri[i] = 1.0 / (i == 1 ? b : b - a * cp[i - 1]);
+    ap[i] = i == 1 ? a * ri[i] : -a * ap[i - 1] * ri[i];
+    cp[i] = c * ri[i];
+  }
+  std::vector<double> fa(ch), fc(ch), r0(ch), la(ch), lc(ch), ra(ch), rc(ch), inv(ch);
+  for (int k = 0; k < ch; k++) {
+    const int m = std::min(R, nx - 2 - k * R);  // real rows; identity rows past them
+    double ab = m > R - 2 ? ap[R - 2] : 0, cb = m > R - 2 ? cp[R - 2] : 0;
+    for (int i = R - 3; i >= 1; i--) {
+      const double ai = i < m ? ap[i] : 0, ci = i < m ? cp[i] : 0;
+      ab = ai - ci * ab;
+      cb = -ci * cb;
+    }
+    r0[k] = 1.0 / (b - c * ab);
+    fa[k] = a * r0[k];
+    fc[k] = -c * cb * r0[k];
+    la[k] = m == R ? ap[R - 1] : 0;
+    lc[k] = m == R ? cp[R - 1] : 0;
+  }
+  const int lv = lines_levels(ch);
+  F.assign((size_t)(6 + 3 * lv) * ch, T(0));
+  auto put = [&](int i, const std::vector<double> &v) {
+    for (int k = 0; k < ch; k++) F[(size_t)i * ch + k] = (T)v[k];
+  };
+  for (int k = 0; k < ch; k++) {
+    const double fna = k + 1 < ch ? fa[k + 1] : 0, fnc = k + 1 < ch ? fc[k + 1] : 0;
+    inv[k] = 1.0 / (1.0 - la[k] * fc[k] - lc[k] * fna);
+    ra[k] = -la[k] * fa[k] * inv[k];
+    rc[k] = -lc[k] * fnc * inv[k];
+  }
+  put(0, r0);
+  put(1, fa);
+  put(2, fc);
+  put(3, la);
+  put(4, lc);
+  put(5, inv);
+  for (int j = 0, s = 1; s < ch; j++, s <<= 1) {
+    std::vector<double> na(ch), nc(ch);
+    for (int k = 0; k < ch; k++) {
+      const double ma = k >= s ? ra[k - s] : 0, mc = k >= s ? rc[k - s] : 0;
+      const double pa = k + s < ch ? ra[k + s] : 0, pc = k + s < ch ? rc[k + s] : 0;
+      inv[k] = 1.0 / (1.0 - ra[k] * mc - rc[k] * pa);
+      na[k] = -ra[k] * ma * inv[k];
+      nc[k] = -rc[k] * pc * inv[k];
+    }
+    put(6 + 3 * j, ra);
+    put(7 + 3 * j, rc);
+    put(8 + 3 * j, inv);
+    ra = na;
+    rc = nc;
+  }
+}
+
+// Builds the plan's factors and queues the copy of the device table (from
+// pageable memory, so the values are taken before it returns); the caller
+// waits for it.  A grid that does not fit leaves lines.R = 0.
+template <typename T>
+tridStatus_t lines_build(tridAdiPlan_st *p) {
+  p->lines = lines_layout(p->nx, p->ny, p->nz, sizeof(T));
+  if (!p->lines.R) return TRID_STATUS_SUCCESS;
+  std::vector<T> F;
+  lines_factors<T>(coefs<T>(p), p->nx, p->lines, p->lines_f[0], p->lines_f[1], p->lines_f[2], F);
+  const size_t bytes = F.size() * sizeof(T);
+  tridStatus_t s = check_hip(hipMalloc(&p->lines_F, bytes), "hipMalloc");
+  hipStream_t st = current_stream();
+  if (!s)
+    s = check_hip(hipMemcpyAsync(p->lines_F, F.data(), bytes, hipMemcpyHostToDevice, st),
+                  "hipMemcpyAsync");
+  if (s) {
+    p->lines.R = 0;
+    (void)hipGetLastError();
+  }
+  return s;
+}
+
+template <typename T, int R, int NP>
+hipError_t launch_lines_t(const tridAdiPlan_st *p, const T *u, T *du, hipStream_t st) {
+  const LinesLayout &L = p->lines;
+  const CoefConst<T> cf = coefs<T>(p);
+  LineFactors<T, R> lf;
+  lf.a = cf.a;
+  lf.c = cf.c;
+  for (int i = 0; i < R; i++) {
+    lf.ri[i] = (T)p->lines_f[0][i];
+    lf.ap[i] = (T)p->lines_f[1][i];
+    lf.cp[i] = (T)p->lines_f[2][i];
+  }
+  lf.F = static_cast<const T *>(p->lines_F);
+  const unsigned nlines = (unsigned)p->ny * (unsigned)p->nz;
+  const unsigned blocks = (nlines + 4u * L.lpw - 1) / (4u * L.lpw);
+  // XCD-contiguous lines while the step's arrays stay in the last-level cache
+  // (the neighbour lines' re-reads then hit the XCD's own L2: 200 x 150 x 180
+  // FP32 50.0 against 53.1 us per step, 250^3 FP64 170 against 193); past it
+  // the plain order is faster (300^3 FP64 387 against 394)
+  const int xcd = p->cp == kCached;
+  if (p->cp == kCached)
+    return launch_kernel(k_adi_rhs_xl<T, R, NP, kCached>, dim3(blocks), dim3(256), 0u, st, u, du,
+                         nlines * (unsigned)p->nx, p->nx, p->ny, p->nz, (T)p->lambda, lf, L.ch,
+                         L.lpw, xcd);
+  return launch_kernel(k_adi_rhs_xl<T, R, NP, kStream>, dim3(blocks), dim3(256), 0u, st, u, du,
+                       nlines * (unsigned)p->nx, p->nx, p->ny, p->nz, (T)p->lambda, lf, L.ch,
+                       L.lpw, xcd);
+}
+
+template <typename T>
+hipError_t launch_lines(const tridAdiPlan_st *p, const T *u, T *du, hipStream_t st) {
+  constexpr int E = Vec16<T>::n;
+#define TRID_LINES(RR)                                                        \
+  if (p->lines.R == RR) {                                                     \
+    constexpr int np = (RR + E - 1) / E;                                      \
+    return p->lines.np == np ? launch_lines_t<T, RR, np>(p, u, du, st)        \
+                             : launch_lines_t<T, RR, np - 1>(p, u, du, st);   \
+  }
+  TRID_LINES(5)
+  TRID_LINES(7)
+  TRID_LINES(9)
+  TRID_LINES(11)
+  TRID_LINES(13)
+#undef TRID_LINES
+  return hipErrorInvalidValue;
+}
+
 // Factor-reuse sweeps: chunk length R in {8, 16, 32} with at most 16 chunks
 // per system (work-groups of 64 systems x cps chunks).
 bool cc_rows_ok(int N, int R, int *cps_log2) {
@@ -503,9 +848,10 @@ bool cc_pair_fits(int R, int cps_log2) {
 }
 
 // Builds the factor table of direction dir for chunk length R into *F
-// (allocated here; waits for the setup kernel).
+// (allocated here; waits for the setup kernel unless the caller does).
 template <typename T>
-tridStatus_t cc_build(tridAdiPlan_st *p, int dir, int R, void **F, int *cps_log2) {
+tridStatus_t cc_build(tridAdiPlan_st *p, int dir, int R, void **F, int *cps_log2,
+                      bool wait = true) {
   const int N = p->desc[dir].N;
   if (!cc_rows_ok(N, R, cps_log2)) return fail(TRID_STATUS_INVALID_VALUE, "cc layout");
   const int cps = 1 << *cps_log2;
@@ -528,7 +874,7 @@ tridStatus_t cc_build(tridAdiPlan_st *p, int dir, int R, void **F, int *cps_log2
     hipLaunchKernelGGL((k_cc_setup<T, 32>), dim3(1), dim3(kWave), 0, st, cf, N, *cps_log2,
                        static_cast<T *>(*F));
   s = check_hip(hipGetLastError(), "factor setup launch");
-  if (!s) s = check_hip(hipStreamSynchronize(st), "hipStreamSynchronize");
+  if (!s && wait) s = check_hip(hipStreamSynchronize(st), "hipStreamSynchronize");
   if (s) {
     (void)hipFree(*F);
     *F = nullptr;
@@ -633,13 +979,19 @@ hipError_t launch_cc(const tridAdiPlan_st *p, int dir, T *d, T *u, hipStream_t s
                              p->cc_F[dir], p->desc[dir], p->cfg[dir].idx32, p->cp, d, u, st);
 }
 
-// Stage 4 = fused RHS + x sweep (plans with fused_R > 0 only).
+// Stage 4 = fused RHS + x sweep (plans with fused_R > 0 only); kLinesStage
+// the whole-line one (lines_R > 0), which tridAdiStep takes where the fused
+// one does not apply.
+constexpr int kLinesStage = 5;
+
 template <typename T>
 tridStatus_t stage_t(tridAdiPlan_st *p, T *u, T *du, int stage, hipStream_t st) {
   hipError_t e = hipSuccess;
   const CoefConst<T> cf = coefs<T>(p);
   if (stage == 4) {
     e = launch_fused<T>(p, u, du, st);
+  } else if (stage == kLinesStage) {
+    e = launch_lines<T>(p, u, du, st);
   } else if (stage == 0) {
     dim3 grid((p->nx + 63) / 64, (p->ny + 3) / 4, (p->nz + kRhsPlanes - 1) / kRhsPlanes);
     if (p->cp == kCached)
@@ -675,11 +1027,17 @@ bool use_fused(const tridAdiPlan_st *p, const void *u, const void *du) {
   return p->fused_R > 0 && aligned16(u) && aligned16(du);
 }
 
+// The whole-line RHS + x kernel serves every grid it fits that the fused
+// kernel does not, and those where it is the faster one (lines_first).
+bool use_lines(const tridAdiPlan_st *p, const void *u, const void *du) {
+  return p->lines.R > 0 && (p->lines_first || !use_fused(p, u, du));
+}
+
 tridStatus_t steps_any(tridAdiPlan_st *p, void *u, void *du, int nsteps, hipStream_t st) {
-  const bool fused = use_fused(p, u, du);
+  const bool lines = use_lines(p, u, du), fused = lines || use_fused(p, u, du);
   for (int s = 0; s < nsteps; s++) {
     if (fused) {
-      for (int g : {4, 2, 3}) {
+      for (int g : {lines ? kLinesStage : 4, 2, 3}) {
         tridStatus_t r = stage_any(p, u, du, g, st);
         if (r) return r;
       }
@@ -787,7 +1145,9 @@ void tune_plan_t(tridAdiPlan_st *p, T *u, T *du) {
   const int n[3] = {p->nx, p->ny, p->nz};
   auto stage = [&](int g) { (void)stage_t<T>(p, u, du, g, st); };
   auto x_stage = [&]() {
-    if (use_fused(p, u, du)) {
+    if (use_lines(p, u, du)) {
+      stage(kLinesStage);
+    } else if (use_fused(p, u, du)) {
       stage(4);
     } else {
       stage(0);
@@ -892,25 +1252,28 @@ void tune_plan_t(tridAdiPlan_st *p, T *u, T *du) {
   // kernel (the untuned choice first)
   if (p->fused_R) {
     struct FusedChoice {
-      int R, xcd, cc;
+      int R, xcd, cc, lines;
     };
-    std::vector<FusedChoice> ch{{p->fused_R, p->fused_xcd, p->fused_cc}};
+    const bool has_lines = p->lines.R > 0;
+    std::vector<FusedChoice> ch{{p->fused_R, p->fused_xcd, p->fused_cc, p->lines_first}};
+    if (has_lines) ch.push_back({p->fused_R, p->fused_xcd, p->fused_cc, !p->lines_first});
     for (int cc : {1, 0})
       for (int R : {4, 8, 16})
         for (int x : {0, 1}) {
           if (!fused_rows_ok(p, R)) continue;
           if (R == p->fused_R && x == p->fused_xcd && cc == p->fused_cc) continue;
           if (cc && fused_table<T>(p, R) != TRID_STATUS_SUCCESS) continue;
-          ch.push_back({R, x, cc});
+          ch.push_back({R, x, cc, 0});
         }
     auto apply = [&](const FusedChoice &c) {
+      p->lines_first = c.lines;
       set_fused(p, c.R);
       p->fused_xcd = c.xcd;
       p->fused_cc = c.cc;
     };
     auto cand = [&](int i) {
       apply(ch[i]);
-      return launch_fused<T>(p, u, du, st);
+      return ch[i].lines ? launch_lines<T>(p, u, du, st) : launch_fused<T>(p, u, du, st);
     };
     auto suffix = [&]() {
       stage(2);
@@ -920,7 +1283,8 @@ void tune_plan_t(tridAdiPlan_st *p, T *u, T *du) {
     const int i = pick_in_step((int)ch.size(), []() {}, cand, suffix, st, &tm);
     if (tune_log())
       for (size_t c = 0; c < ch.size(); c++)
-        fprintf(stderr, "[tridhip tune] rhs+x fused R%d%s%s: %.4f ms\n", ch[c].R,
+        fprintf(stderr, "[tridhip tune] rhs+x %s R%d%s%s: %.4f ms\n",
+                ch[c].lines ? "lines" : "fused", ch[c].lines ? p->lines.R : ch[c].R,
                 ch[c].cc ? ",cc" : "", ch[c].xcd ? ",xcd" : "", tm[c]);
     apply(ch[i >= 0 ? i : 0]);
   }
@@ -970,8 +1334,13 @@ std::string plan_text(const tridAdiPlan_st *p) {
   if (p->fused_R)
     fx = "rhs+x(fused,R" + std::to_string(p->fused_R) + (p->fused_cc ? ",cc" : "") +
          (p->fused_xcd ? ",xcd" : "") + cached + ")<";
+  else if (p->lines.R)
+    fx = "rhs+x(lines,R" + std::to_string(p->lines.R) + cached + ")<";
   return fx + (p->dbl ? "double" : "float") + "> x:" + part_name(0) + " y:" + sweep_name(1) +
-         " z:" + sweep_name(2);
+         " z:" + sweep_name(2) +
+         (p->fused_R && p->lines_first
+              ? " step:rhs+x(lines,R" + std::to_string(p->lines.R) + cached + ")"
+              : std::string());
 }
 
 // With autotuning on, a plan tunes at its first use, on that call's arrays,
@@ -1057,14 +1426,22 @@ EXTERN_C tridStatus_t tridAdiPlanCreate(tridAdiPlan_t *plan, int nx, int ny,
         break;
       }
   }
+  (void)(p->dbl ? lines_build<double>(p) : lines_build<float>(p));
+  // FP32 grids the fused kernel takes: the whole-line kernel's precomputed
+  // factors and 16-byte pieces win for lines of 128 and 256 points (256^3
+  // 95.0 against 104.2 us per step, 128 x 300 x 300 102.6 against 110.8); at
+  // 64 points they tie and at 512 its 9-row chunks leave a fifth of the wave
+  // idle (512 x 512 x 128 184 against 170).  In FP64 the fused kernel is 1 %
+  // ahead at 256^3 and level at 128^3.
+  p->lines_first = !p->dbl && p->fused_R && p->lines.R && nx >= 128 && nx <= 256;
   // y and z sweeps: factor reuse by default when a chunk layout fits
   for (int dir = 1; dir < 3; dir++) {
     for (int R : {16, 8, 32}) {
       int cl = 0;
       if (!cc_rows_ok(n[dir], R, &cl)) continue;
       void *F = nullptr;
-      const tridStatus_t r = p->dbl ? cc_build<double>(p, dir, R, &F, &cl)
-                                    : cc_build<float>(p, dir, R, &F, &cl);
+      const tridStatus_t r = p->dbl ? cc_build<double>(p, dir, R, &F, &cl, false)
+                                    : cc_build<float>(p, dir, R, &F, &cl, false);
       if (r == TRID_STATUS_SUCCESS) {
         p->cc_R[dir] = R;
         p->cc_cps_log2[dir] = cl;
@@ -1072,6 +1449,17 @@ EXTERN_C tridStatus_t tridAdiPlanCreate(tridAdiPlan_t *plan, int nx, int ny,
         p->cc_F[dir] = F;
       }
       break;
+    }
+  }
+  // one wait for the three tables; without them the plan runs the generic
+  // sweeps
+  if (hipStreamSynchronize(current_stream()) != hipSuccess) {
+    (void)hipGetLastError();
+    p->lines.R = p->lines_first = 0;
+    for (int dir = 1; dir < 3; dir++) {
+      if (p->cc_F[dir]) (void)hipFree(p->cc_F[dir]);
+      p->cc_F[dir] = nullptr;
+      p->cc_R[dir] = 0;
     }
   }
   clear_error();
@@ -1143,6 +1531,7 @@ EXTERN_C tridStatus_t tridAdiPlanDestroy(tridAdiPlan_t p) {
     if (F) (void)hipFree(F);
   for (void *F : p->fused_F)
     if (F) (void)hipFree(F);
+  if (p->lines_F) (void)hipFree(p->lines_F);
   delete p;
   return TRID_STATUS_SUCCESS;
 }
@@ -1249,6 +1638,7 @@ EXTERN_C tridStatus_t tridAdiPlanSetSweep(tridAdiPlan_t p, int dir, int rows, in
     set_fused(p, rows);
     p->fused_xcd = xcd;
     p->fused_cc = pair;
+    p->lines_first = 0;
     p->tune_pending = false;
     p->text = plan_text(p);
     clear_error();
