@@ -95,3 +95,23 @@ def test_adi_lines_autotuned():
         assert oracle.rel_err(exp, u.cpu().numpy().ravel()) <= tol(dt), plan.describe()
         plan.set_sweep(0, 8)
         assert "step:" not in plan.describe()
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("shape", [(256, 300, 130), (256, 130, 300), (190, 128, 180),
+                                   (181, 257, 182), (64, 129, 513)])
+def test_adi_default_sweep_layouts(shape, dt):
+    """The untuned y and z layouts on both sides of their rules: line lengths
+    around 128, 256 and 512 points, batches that fill the work-groups of two
+    lines per lane (32768 lines) or not, odd line counts, chunk counts that are
+    no power of two."""
+    import torch
+    nx, ny, nz = shape
+    u0 = rand_init(nx, ny, nz, dt, seed=ny)
+    exp = u0.ravel().copy()
+    assert oracle.adi(exp, nx, ny, nz, 1, 1.0, 1) == 0
+    plan = AdiPlan(nx, ny, nz, torch_dt(dt))
+    u = torch.from_numpy(u0).cuda()
+    plan.step(u, torch.empty_like(u), 1)
+    err = oracle.rel_err(exp, u.cpu().numpy().ravel())
+    assert err <= tol(dt), f"{err:.2e} [{plan.describe()}]"

@@ -512,6 +512,91 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+constexpr int kLinesMaxRows = 13;
+
+// What k_lines_setup needs of the interior matrix: its coefficients and the
+// rows after the forward sweep of a chunk.
+struct LineRows {
+  double a, b, c;
+  double ap[kLinesMaxRows], cp[kLinesMaxRows];
+};
+
+// The per-chunk factors of k_adi_rhs_xl (LineFactors::F) for chunks of R rows
+// and ch <= 64 chunks: the recurrences of chunk_reduce, eliminate_first and
+// pcr_update on the coefficients, in double.  One wave, thread k chunk k.
+template <typename T>
+__device__ __forceinline__ void lines_setup_wave(const LineRows &lr, int R, int nx, int ch,
+                                                 T *__restrict__ F, double *sa, double *sc) {
+  const int k = threadIdx.x;
+  const bool on = k < ch;
+  auto put = [&](int i, double v) {
+    if (on) F[i * ch + k] = (T)v;
+  };
+  const int left = nx - 2 - k * R, m = left < R ? left : R;  // real rows; identity past them
+  double ab = m > R - 2 ? lr.ap[R - 2] : 0.0, cb = m > R - 2 ? lr.cp[R - 2] : 0.0;
+  for (int i = R - 3; i >= 1; i--) {
+    const double ai = i < m ? lr.ap[i] : 0.0, ci = i < m ? lr.cp[i] : 0.0;
+    ab = ai - ci * ab;
+    cb = -ci * cb;
+  }
+  const double r0 = 1.0 / (lr.b - lr.c * ab);
+  const double fa = lr.a * r0, fc = -lr.c * cb * r0;
+  const double la = m == R ? lr.ap[R - 1] : 0.0, lc = m == R ? lr.cp[R - 1] : 0.0;
+  put(0, r0);
+  put(1, fa);
+  put(2, fc);
+  put(3, la);
+  put(4, lc);
+  sa[k] = on ? fa : 0.0;
+  sc[k] = on ? fc : 0.0;
+  __syncthreads();
+  const double fna = k + 1 < ch ? sa[k + 1] : 0.0, fnc = k + 1 < ch ? sc[k + 1] : 0.0;
+  double inv = 1.0 / (1.0 - la * fc - lc * fna);
+  put(5, inv);
+  double ra = -la * fa * inv, rc = -lc * fnc * inv;
+  for (int j = 6, s = 1; s < ch; j += 3, s <<= 1) {
+    __syncthreads();
+    sa[k] = on ? ra : 0.0;
+    sc[k] = on ? rc : 0.0;
+    __syncthreads();
+    const double ma = k >= s ? sa[k - s] : 0.0, mc = k >= s ? sc[k - s] : 0.0;
+    const double pa = k + s < ch ? sa[k + s] : 0.0, pc = k + s < ch ? sc[k + s] : 0.0;
+    inv = 1.0 / (1.0 - ra * mc - rc * pa);
+    put(j, ra);
+    put(j + 1, rc);
+    put(j + 2, inv);
+    ra = -ra * ma * inv;
+    rc = -rc * pc * inv;
+  }
+}
+
+// The tables of a new plan in one launch: work-group 0 the whole-line x
+// sweep's, 1 and 2 the y and z sweeps' (R = 0: none).
+struct TableJob {
+  int R = 0, N = 0, chunks = 0;
+  void *F = nullptr;
+};
+struct TableJobs {
+  TableJob job[3];
+};
+template <typename T>
+__global__ void __launch_bounds__(kWave)
+    k_adi_tables(LineRows lr, CoefConst<T> cf, TableJobs jobs) {
+  __shared__ double sa[kWave], sc[kWave];
+  const int b = blockIdx.x;
+  const TableJob j = jobs.job[b];
+  T *F = static_cast<T *>(j.F), *ta = reinterpret_cast<T *>(sa), *tc = reinterpret_cast<T *>(sc);
+  if (j.R == 0) return;
+  if (b == 0)
+    lines_setup_wave<T>(lr, j.R, j.N, j.chunks, F, sa, sc);
+  else if (j.R == 8)
+    cc_setup_wave<T, 8>(cf, j.N, j.chunks, F, ta, tc);
+  else if (j.R == 16)
+    cc_setup_wave<T, 16>(cf, j.N, j.chunks, F, ta, tc);
+  else
+    cc_setup_wave<T, 32>(cf, j.N, j.chunks, F, ta, tc);
+}
+
 namespace {
 
 SysDesc grid_desc(int nx, int ny, int nz, int dir) {
@@ -561,17 +646,21 @@ struct tridAdiPlan_st {
   int fused_cc = 0;         // fused x sweep with precomputed factors
   void *fused_F[3] = {nullptr, nullptr, nullptr};  // their tables, chunk length 4, 8, 16
   LinesLayout lines;        // R > 0: whole-line RHS + x sweep and its factors
-  double lines_f[3][16] = {};  // per-row factors ri, ap, cp
-  void *lines_F = nullptr;     // per-chunk factors (device)
+  double lines_f[3][kLinesMaxRows] = {};  // per-row factors ri, ap, cp
+  void *lines_F = nullptr;     // per-chunk factors (device, in `tables`)
   int lines_first = 0;         // tridAdiStep prefers it to the fused kernel
   int cp = 0;               // cache policy of every stage's streaming accesses
   // y and z sweeps with precomputed factors (trid_cc.hpp): chunk length (0 =
   // the generic kernel), chunks per system and the factor table
   int cc_R[3] = {0, 0, 0};
-  int cc_cps_log2[3] = {0, 0, 0};
+  int cc_cps[3] = {0, 0, 0};
   int cc_xcd[3] = {0, 0, 0};
   int cc_pair[3] = {0, 0, 0};  // two adjacent systems per lane (16-byte rows)
   void *cc_F[3] = {nullptr, nullptr, nullptr};
+  // one allocation for the tables the plan is created with (lines_F and the
+  // first cc_F); later cc_F are their own allocations
+  void *tables = nullptr;
+  bool cc_own[3] = {false, false, false};
   bool tune_pending = false;
   hipGraph_t graph = nullptr;  // tridAdiGraphCapture's graph
   hipGraphExec_t exec = nullptr;
@@ -664,7 +753,7 @@ hipError_t launch_fused(tridAdiPlan_st *p, T *u, T *du, hipStream_t st) {
   return hipGetLastError();
 }
 
-constexpr int kLinesRows[] = {5, 7, 9, 11, 13};
+constexpr int kLinesRows[] = {5, 7, 9, 11, kLinesMaxRows};
 
 LinesLayout lines_layout(int nx, int ny, int nz, size_t tsize) {
   LinesLayout best;
@@ -694,92 +783,18 @@ LinesLayout lines_layout(int nx, int ny, int nz, size_t tsize) {
   return best;
 }
 
-// Levels of the reduced system's PCR over ch chunks.
-int lines_levels(int ch) { return ilog2(ch); }
-
-// The factors of the whole-line x sweep: the recurrences of chunk_reduce,
-// eliminate_first and pcr_update on the coefficients, in double.  Per-row
-// factors to ri, ap, cp (R values each), per-chunk ones to F.
+// Per-row factors of the plan's whole-line x sweep, from the interior matrix
+// in double.
 template <typename T>
-void lines_factors(const CoefConst<T> &cf, int nx, const LinesLayout &L, double *ri, double *ap,
-                   double *cp, std::vector<T> &F) {
+void lines_rows(tridAdiPlan_st *p) {
+  const CoefConst<T> cf = coefs<T>(p);
   const double a = cf.a, b = cf.b, c = cf.c;
-  const int R = L.R, ch = L.ch;
-  ri[0] = ap[0] = cp[0] = 0;
-  for (int i = 1; i < R; i++) {
+  double *ri = p->lines_f[0], *ap = p->lines_f[1], *cp = p->lines_f[2];
+  for (int i = 1; i < p->lines.R; i++) {
     ri[i] = 1.0 / (i == 1 ? b : b - a * cp[i - 1]);
     ap[i] = i == 1 ? a * ri[i] : -a * ap[i - 1] * ri[i];
     cp[i] = c * ri[i];
   }
-  std::vector<double> fa(ch), fc(ch), r0(ch), la(ch), lc(ch), ra(ch), rc(ch), inv(ch);
-  for (int k = 0; k < ch; k++) {
-    const int m = std::min(R, nx - 2 - k * R);  // real rows; identity rows past them
-    double ab = m > R - 2 ? ap[R - 2] : 0, cb = m > R - 2 ? cp[R - 2] : 0;
-    for (int i = R - 3; i >= 1; i--) {
-      const double ai = i < m ? ap[i] : 0, ci = i < m ? cp[i] : 0;
-      ab = ai - ci * ab;
-      cb = -ci * cb;
-    }
-    r0[k] = 1.0 / (b - c * ab);
-    fa[k] = a * r0[k];
-    fc[k] = -c * cb * r0[k];
-    la[k] = m == R ? ap[R - 1] : 0;
-    lc[k] = m == R ? cp[R - 1] : 0;
-  }
-  const int lv = lines_levels(ch);
-  F.assign((size_t)(6 + 3 * lv) * ch, T(0));
-  auto put = [&](int i, const std::vector<double> &v) {
-    for (int k = 0; k < ch; k++) F[(size_t)i * ch + k] = (T)v[k];
-  };
-  for (int k = 0; k < ch; k++) {
-    const double fna = k + 1 < ch ? fa[k + 1] : 0, fnc = k + 1 < ch ? fc[k + 1] : 0;
-    inv[k] = 1.0 / (1.0 - la[k] * fc[k] - lc[k] * fna);
-    ra[k] = -la[k] * fa[k] * inv[k];
-    rc[k] = -lc[k] * fnc * inv[k];
-  }
-  put(0, r0);
-  put(1, fa);
-  put(2, fc);
-  put(3, la);
-  put(4, lc);
-  put(5, inv);
-  for (int j = 0, s = 1; s < ch; j++, s <<= 1) {
-    std::vector<double> na(ch), nc(ch);
-    for (int k = 0; k < ch; k++) {
-      const double ma = k >= s ? ra[k - s] : 0, mc = k >= s ? rc[k - s] : 0;
-      const double pa = k + s < ch ? ra[k + s] : 0, pc = k + s < ch ? rc[k + s] : 0;
-      inv[k] = 1.0 / (1.0 - ra[k] * mc - rc[k] * pa);
-      na[k] = -ra[k] * ma * inv[k];
-      nc[k] = -rc[k] * pc * inv[k];
-    }
-    put(6 + 3 * j, ra);
-    put(7 + 3 * j, rc);
-    put(8 + 3 * j, inv);
-    ra = na;
-    rc = nc;
-  }
-}
-
-// Builds the plan's factors and queues the copy of the device table (from
-// pageable memory, so the values are taken before it returns); the caller
-// waits for it.  A grid that does not fit leaves lines.R = 0.
-template <typename T>
-tridStatus_t lines_build(tridAdiPlan_st *p) {
-  p->lines = lines_layout(p->nx, p->ny, p->nz, sizeof(T));
-  if (!p->lines.R) return TRID_STATUS_SUCCESS;
-  std::vector<T> F;
-  lines_factors<T>(coefs<T>(p), p->nx, p->lines, p->lines_f[0], p->lines_f[1], p->lines_f[2], F);
-  const size_t bytes = F.size() * sizeof(T);
-  tridStatus_t s = check_hip(hipMalloc(&p->lines_F, bytes), "hipMalloc");
-  hipStream_t st = current_stream();
-  if (!s)
-    s = check_hip(hipMemcpyAsync(p->lines_F, F.data(), bytes, hipMemcpyHostToDevice, st),
-                  "hipMemcpyAsync");
-  if (s) {
-    p->lines.R = 0;
-    (void)hipGetLastError();
-  }
-  return s;
 }
 
 template <typename T, int R, int NP>
@@ -831,55 +846,132 @@ hipError_t launch_lines(const tridAdiPlan_st *p, const T *u, T *du, hipStream_t 
 
 // Factor-reuse sweeps: chunk length R in {8, 16, 32} with at most 16 chunks
 // per system (work-groups of 64 systems x cps chunks).
-bool cc_rows_ok(int N, int R, int *cps_log2) {
+bool cc_rows_ok(int N, int R, int *cps) {
   if (R != 8 && R != 16 && R != 32) return false;
   const long long ch = (N + R - 1) / R;
-  int cl = 0;
-  while ((1LL << cl) < ch) cl++;
-  if ((kWave << cl) > cc_max_threads(R, 1)) return false;
-  *cps_log2 = cl;
+  if (kWave * ch > cc_max_threads(R, 1, 8, 8)) return false;
+  *cps = (int)ch;
   return true;
 }
 
-// Two systems per lane fit chunk lengths up to 32 rows in work-groups within
-// the kernel's launch bound.
-bool cc_pair_fits(int R, int cps_log2) {
-  return R <= 32 && (kWave << cps_log2) <= cc_max_threads(R, 2);
+// Two systems per lane fit work-groups within the kernel's launch bound.
+bool cc_pair_fits(const tridAdiPlan_st *p, int R, int cps) {
+  return kWave * cps <= cc_max_threads(R, 2, p->dbl ? 8 : 4, p->cfg[1].idx32 ? 4 : 8);
+}
+
+// Untuned layout of the factor-reuse sweep of direction dir, from step times
+// on 27 grids (MI355X): rows, two lines per lane and the XCD-contiguous order.
+//   pair: where the 128-line work-groups still fill the 256 CUs, else one line
+//     per lane (128^3 FP64 z 16.4 -> 11.6 us with 8-row chunks; 200 x 150 x
+//     180 FP32 z -3.2 us of 46).  Wide rows carry the long lines: 512^3 FP32
+//     z 302 -> 185 us, 300^3 -25 of 203.
+//   rows: 8 up to 128-row lines (FP64 pairs 16: 256 x 256 x 128 z -2.7 us),
+//     16 up to 256, else 32.
+//   xcd: y always (512^3 FP64 -104 us of 1708, 200 x 150 x 180 FP32 -1.2 of
+//     46: the lines of a work-group and of the next share row ends); z while
+//     the arrays stay in the last-level cache (256^3 FP64 -9 us of 170; past
+//     it 512 x 512 x 128 FP64 +23 of 392).
+struct CCChoice {
+  int R, cps, pair, xcd;
+};
+bool cc_default(const tridAdiPlan_st *p, int dir, CCChoice *c) {
+  const SysDesc &D = p->desc[dir];
+  const bool wide = D.osize[0] % 2 == 0 && D.nsys >= 256LL * 2 * kWave;
+  c->R = D.N > 256 ? 32 : (D.N > 128 || (p->dbl && wide) ? 16 : 8);
+  if (!cc_rows_ok(D.N, c->R, &c->cps)) return false;
+  c->pair = wide && cc_pair_fits(p, c->R, c->cps);
+  c->xcd = dir == 1 || p->cp == kCached;
+  return true;
+}
+
+size_t cc_table_bytes(int R, int cps, size_t tsize) {
+  const int lv = cc_levels(cps);
+  const int nf = R == 8 ? CCLayout<8>::nf(lv) : (R == 16 ? CCLayout<16>::nf(lv)
+                                                         : CCLayout<32>::nf(lv));
+  return (size_t)cps * nf * tsize;
 }
 
 // Builds the factor table of direction dir for chunk length R into *F
-// (allocated here; waits for the setup kernel unless the caller does).
+// (allocated here; waits for the setup kernel).
 template <typename T>
-tridStatus_t cc_build(tridAdiPlan_st *p, int dir, int R, void **F, int *cps_log2,
-                      bool wait = true) {
+tridStatus_t cc_build(tridAdiPlan_st *p, int dir, int R, void **F, int *ncps) {
   const int N = p->desc[dir].N;
-  if (!cc_rows_ok(N, R, cps_log2)) return fail(TRID_STATUS_INVALID_VALUE, "cc layout");
-  const int cps = 1 << *cps_log2;
-  size_t nf = 0;
-  if (R == 8) nf = CCLayout<8>::nf(*cps_log2);
-  else if (R == 16) nf = CCLayout<16>::nf(*cps_log2);
-  else nf = CCLayout<32>::nf(*cps_log2);
-  tridStatus_t s = check_hip(hipMalloc(F, cps * nf * sizeof(T)), "hipMalloc");
+  if (!cc_rows_ok(N, R, ncps)) return fail(TRID_STATUS_INVALID_VALUE, "cc layout");
+  tridStatus_t s = check_hip(hipMalloc(F, cc_table_bytes(R, *ncps, sizeof(T))), "hipMalloc");
   if (s) return s;
-  const CoefConst<T> cf = coefs<T>(p);
-  // one wave (cps <= 16)
+  TableJobs jobs;
+  jobs.job[1] = {R, N, *ncps, *F};
   hipStream_t st = current_stream();
-  if (R == 8)
-    hipLaunchKernelGGL((k_cc_setup<T, 8>), dim3(1), dim3(kWave), 0, st, cf, N, *cps_log2,
-                       static_cast<T *>(*F));
-  else if (R == 16)
-    hipLaunchKernelGGL((k_cc_setup<T, 16>), dim3(1), dim3(kWave), 0, st, cf, N, *cps_log2,
-                       static_cast<T *>(*F));
-  else
-    hipLaunchKernelGGL((k_cc_setup<T, 32>), dim3(1), dim3(kWave), 0, st, cf, N, *cps_log2,
-                       static_cast<T *>(*F));
+  hipLaunchKernelGGL(k_adi_tables<T>, dim3(2), dim3(kWave), 0, st, LineRows{}, coefs<T>(p), jobs);
   s = check_hip(hipGetLastError(), "factor setup launch");
-  if (!s && wait) s = check_hip(hipStreamSynchronize(st), "hipStreamSynchronize");
+  if (!s) s = check_hip(hipStreamSynchronize(st), "hipStreamSynchronize");
   if (s) {
     (void)hipFree(*F);
     *F = nullptr;
   }
   return s;
+}
+
+// Replaces the table of direction dir (the plan then owns F).
+void cc_replace(tridAdiPlan_st *p, int dir, void *F) {
+  if (p->cc_own[dir] && p->cc_F[dir]) (void)hipFree(p->cc_F[dir]);
+  p->cc_F[dir] = F;
+  p->cc_own[dir] = true;
+}
+
+// The tables of a new plan: the whole-line x sweep's and the default y and z
+// sweeps', in one allocation with one wait.  Without them (no memory, a
+// failed launch) the plan runs the generic kernels.
+template <typename T>
+void build_tables(tridAdiPlan_st *p) {
+  p->lines = lines_layout(p->nx, p->ny, p->nz, sizeof(T));
+  if (p->lines.R) lines_rows<T>(p);
+  CCChoice c[3];
+  bool cc[3] = {false, false, false};
+  size_t off[4] = {0, 0, 0, 0};  // byte offsets of the three tables and the end
+  if (p->lines.R)
+    off[1] = ((6 + 3 * cc_levels(p->lines.ch)) * p->lines.ch * sizeof(T) + 255) / 256 * 256;
+  for (int dir = 1; dir < 3; dir++) {
+    cc[dir] = cc_default(p, dir, &c[dir]);
+    off[dir + 1] =
+        off[dir] + (cc[dir] ? (cc_table_bytes(c[dir].R, c[dir].cps, sizeof(T)) + 255) / 256 * 256
+                            : 0);
+  }
+  if (!off[3]) return;
+  hipStream_t st = current_stream();
+  bool ok = hipMalloc(&p->tables, off[3]) == hipSuccess;
+  char *base = static_cast<char *>(p->tables);
+  if (ok) {
+    LineRows lr{};
+    TableJobs jobs;
+    const CoefConst<T> cf = coefs<T>(p);
+    if (p->lines.R) {
+      lr.a = cf.a;
+      lr.b = cf.b;
+      lr.c = cf.c;
+      std::copy(p->lines_f[1], p->lines_f[1] + kLinesMaxRows, lr.ap);
+      std::copy(p->lines_f[2], p->lines_f[2] + kLinesMaxRows, lr.cp);
+      jobs.job[0] = {p->lines.R, p->nx, p->lines.ch, base};
+    }
+    for (int dir = 1; dir < 3; dir++)
+      if (cc[dir]) jobs.job[dir] = {c[dir].R, p->desc[dir].N, c[dir].cps, base + off[dir]};
+    hipLaunchKernelGGL(k_adi_tables<T>, dim3(3), dim3(kWave), 0, st, lr, cf, jobs);
+    ok = hipGetLastError() == hipSuccess && hipStreamSynchronize(st) == hipSuccess;
+  }
+  if (!ok) {
+    (void)hipGetLastError();
+    p->lines.R = 0;
+    return;
+  }
+  p->lines_F = base;
+  for (int dir = 1; dir < 3; dir++)
+    if (cc[dir]) {
+      p->cc_R[dir] = c[dir].R;
+      p->cc_cps[dir] = c[dir].cps;
+      p->cc_pair[dir] = c[dir].pair;  // used when the arrays allow it (cc_pair_ok)
+      p->cc_xcd[dir] = c[dir].xcd;
+      p->cc_F[dir] = base + off[dir];
+    }
 }
 
 // Factor table of the fused x sweep with chunk length R (fused_rows_ok(p, R)
@@ -900,11 +992,11 @@ tridStatus_t fused_table(tridAdiPlan_st *p, int R) {
   hipStream_t st = current_stream();
   T *f = static_cast<T *>(F);
   if (R == 4)
-    hipLaunchKernelGGL((k_cc_setup<T, 4>), dim3(1), dim3(kWave), 0, st, cf, p->nx, cl, f);
+    hipLaunchKernelGGL((k_cc_setup<T, 4>), dim3(1), dim3(kWave), 0, st, cf, p->nx, cps, f);
   else if (R == 8)
-    hipLaunchKernelGGL((k_cc_setup<T, 8>), dim3(1), dim3(kWave), 0, st, cf, p->nx, cl, f);
+    hipLaunchKernelGGL((k_cc_setup<T, 8>), dim3(1), dim3(kWave), 0, st, cf, p->nx, cps, f);
   else
-    hipLaunchKernelGGL((k_cc_setup<T, 16>), dim3(1), dim3(kWave), 0, st, cf, p->nx, cl, f);
+    hipLaunchKernelGGL((k_cc_setup<T, 16>), dim3(1), dim3(kWave), 0, st, cf, p->nx, cps, f);
   s = check_hip(hipGetLastError(), "factor setup launch");
   if (!s) s = check_hip(hipStreamSynchronize(st), "hipStreamSynchronize");
   if (s) {
@@ -929,9 +1021,8 @@ bool cc_pair_ok(const SysDesc &D, const T *d, const T *u, int inc) {
 }
 
 template <typename T, int INC>
-hipError_t launch_cc_t(int R, int cps_log2, int xcd, int pair, const void *F, const SysDesc &D,
+hipError_t launch_cc_t(int R, int cps, int xcd, int pair, const void *F, const SysDesc &D,
                        int idx32, int cp, T *d, T *u, hipStream_t st) {
-  const int cps = 1 << cps_log2;
   const int ns = pair ? 2 : 1;
   const long long per = (long long)kWave * ns;
   const unsigned blocks = (unsigned)((D.nsys + per - 1) / per);
@@ -940,7 +1031,7 @@ hipError_t launch_cc_t(int R, int cps_log2, int xcd, int pair, const void *F, co
   const T *f = static_cast<const T *>(F);
 #define TRID_CC(RR, II, NN, CC)                                                           \
   (void)launch_kernel(k_cc_sweep<T, INC, RR, II, NN, CC>, grid, block, (std::uint32_t)lds, st, \
-                      f, d, u, D, cps_log2, xcd)
+                      f, d, u, D, cps, xcd)
 #define TRID_CC_R(II, NN, CC)             \
   if (R == 8) TRID_CC(8, II, NN, CC);       \
   else if (R == 16) TRID_CC(16, II, NN, CC); \
@@ -973,9 +1064,9 @@ hipError_t launch_cc_t(int R, int cps_log2, int xcd, int pair, const void *F, co
 
 template <typename T, int INC>
 hipError_t launch_cc(const tridAdiPlan_st *p, int dir, T *d, T *u, hipStream_t st) {
-  const int pair = p->cc_pair[dir] && cc_pair_fits(p->cc_R[dir], p->cc_cps_log2[dir]) &&
+  const int pair = p->cc_pair[dir] && cc_pair_fits(p, p->cc_R[dir], p->cc_cps[dir]) &&
                    cc_pair_ok<T>(p->desc[dir], d, u, INC);
-  return launch_cc_t<T, INC>(p->cc_R[dir], p->cc_cps_log2[dir], p->cc_xcd[dir], pair,
+  return launch_cc_t<T, INC>(p->cc_R[dir], p->cc_cps[dir], p->cc_xcd[dir], pair,
                              p->cc_F[dir], p->desc[dir], p->cfg[dir].idx32, p->cp, d, u, st);
 }
 
@@ -1181,8 +1272,7 @@ void tune_plan_t(tridAdiPlan_st *p, T *u, T *du) {
       gen.push_back({0, 0, 0, 0, 0, c, nullptr});
     }
     const bool pair_ok = cc_pair_ok<T>(p->desc[dir], du, u, dir == 2);
-    if (p->cc_F[dir]) (void)hipFree(p->cc_F[dir]);
-    p->cc_F[dir] = nullptr;
+    cc_replace(p, dir, nullptr);
     p->cc_R[dir] = 0;
     std::vector<void *> tables;
     for (int R : {16, 32, 8}) {
@@ -1192,7 +1282,7 @@ void tune_plan_t(tridAdiPlan_st *p, T *u, T *du) {
       if (cc_build<T>(p, dir, R, &F, &cl) != TRID_STATUS_SUCCESS) continue;
       tables.push_back(F);
       // two lines per lane first: the usual winner
-      for (int pr = (pair_ok && cc_pair_fits(R, cl) ? 1 : 0); pr >= 0; pr--) {
+      for (int pr = (pair_ok && cc_pair_fits(p, R, cl) ? 1 : 0); pr >= 0; pr--) {
         fac.push_back({1, R, cl, 0, pr, p->cfg[dir], F});
         fac.push_back({1, R, cl, 1, pr, p->cfg[dir], F});
       }
@@ -1207,7 +1297,7 @@ void tune_plan_t(tridAdiPlan_st *p, T *u, T *du) {
     auto apply = [&](const Choice &c) {
       if (c.cc) {
         p->cc_R[dir] = c.R;
-        p->cc_cps_log2[dir] = c.cl;
+        p->cc_cps[dir] = c.cl;
         p->cc_xcd[dir] = c.xcd;
         p->cc_pair[dir] = c.pair;
         p->cc_F[dir] = c.F;
@@ -1327,7 +1417,7 @@ std::string plan_text(const tridAdiPlan_st *p) {
   auto sweep_name = [&](int dir) {
     if (!p->cc_R[dir]) return part_name(dir);
     return "cc<R" + std::to_string(p->cc_R[dir]) + ",cps" +
-           std::to_string(1 << p->cc_cps_log2[dir]) + (p->cc_xcd[dir] ? ",xcd" : "") +
+           std::to_string(p->cc_cps[dir]) + (p->cc_xcd[dir] ? ",xcd" : "") +
            (p->cc_pair[dir] ? ",pair" : "") + cached + ">";
   };
   std::string fx = "rhs" + cached + "<";
@@ -1426,7 +1516,9 @@ EXTERN_C tridStatus_t tridAdiPlanCreate(tridAdiPlan_t *plan, int nx, int ny,
         break;
       }
   }
-  (void)(p->dbl ? lines_build<double>(p) : lines_build<float>(p));
+  // y and z sweeps: factor reuse by default when a chunk layout fits
+  if (p->dbl) build_tables<double>(p);
+  else build_tables<float>(p);
   // FP32 grids the fused kernel takes: the whole-line kernel's precomputed
   // factors and 16-byte pieces win for lines of 128 and 256 points (256^3
   // 95.0 against 104.2 us per step, 128 x 300 x 300 102.6 against 110.8); at
@@ -1434,34 +1526,6 @@ EXTERN_C tridStatus_t tridAdiPlanCreate(tridAdiPlan_t *plan, int nx, int ny,
   // idle (512 x 512 x 128 184 against 170).  In FP64 the fused kernel is 1 %
   // ahead at 256^3 and level at 128^3.
   p->lines_first = !p->dbl && p->fused_R && p->lines.R && nx >= 128 && nx <= 256;
-  // y and z sweeps: factor reuse by default when a chunk layout fits
-  for (int dir = 1; dir < 3; dir++) {
-    for (int R : {16, 8, 32}) {
-      int cl = 0;
-      if (!cc_rows_ok(n[dir], R, &cl)) continue;
-      void *F = nullptr;
-      const tridStatus_t r = p->dbl ? cc_build<double>(p, dir, R, &F, &cl, false)
-                                    : cc_build<float>(p, dir, R, &F, &cl, false);
-      if (r == TRID_STATUS_SUCCESS) {
-        p->cc_R[dir] = R;
-        p->cc_cps_log2[dir] = cl;
-        p->cc_pair[dir] = cc_pair_fits(R, cl);  // used when the arrays allow it (cc_pair_ok)
-        p->cc_F[dir] = F;
-      }
-      break;
-    }
-  }
-  // one wait for the three tables; without them the plan runs the generic
-  // sweeps
-  if (hipStreamSynchronize(current_stream()) != hipSuccess) {
-    (void)hipGetLastError();
-    p->lines.R = p->lines_first = 0;
-    for (int dir = 1; dir < 3; dir++) {
-      if (p->cc_F[dir]) (void)hipFree(p->cc_F[dir]);
-      p->cc_F[dir] = nullptr;
-      p->cc_R[dir] = 0;
-    }
-  }
   clear_error();
   p->tune_pending = autotune_mode() == 1;
   p->text = plan_text(p);
@@ -1527,11 +1591,10 @@ EXTERN_C tridStatus_t tridAdiPlanDestroy(tridAdiPlan_t p) {
   if (!p) return TRID_STATUS_SUCCESS;
   drop_graphs(p, true);
   if (p->cap) (void)hipStreamDestroy(p->cap);
-  for (void *F : p->cc_F)
-    if (F) (void)hipFree(F);
+  for (int dir = 1; dir < 3; dir++) cc_replace(p, dir, nullptr);
   for (void *F : p->fused_F)
     if (F) (void)hipFree(F);
-  if (p->lines_F) (void)hipFree(p->lines_F);
+  if (p->tables) (void)hipFree(p->tables);
   delete p;
   return TRID_STATUS_SUCCESS;
 }
@@ -1649,7 +1712,7 @@ EXTERN_C tridStatus_t tridAdiPlanSetSweep(tridAdiPlan_t p, int dir, int rows, in
   if (rows != 0) {
     if (!cc_rows_ok(p->desc[dir].N, rows, &cl))
       return fail(TRID_STATUS_INVALID_VALUE, "rows do not fit the line length");
-    if (pair && !cc_pair_fits(rows, cl))
+    if (pair && kWave * cl > cc_max_threads(rows, 2, 8, 8))
       return fail(TRID_STATUS_INVALID_VALUE, "two lines per lane do not fit these rows");
     const tridStatus_t s = p->dbl ? cc_build<double>(p, dir, rows, &F, &cl)
                                   : cc_build<float>(p, dir, rows, &F, &cl);
@@ -1660,10 +1723,9 @@ EXTERN_C tridStatus_t tridAdiPlanSetSweep(tridAdiPlan_t p, int dir, int rows, in
   // graphs hold the old factor table and kernel choice; hipFree waits for
   // queued kernels that may still read the old factors
   drop_graphs(p, true);
-  if (p->cc_F[dir]) (void)hipFree(p->cc_F[dir]);
-  p->cc_F[dir] = F;
+  cc_replace(p, dir, F);
   p->cc_R[dir] = rows;
-  p->cc_cps_log2[dir] = cl;
+  p->cc_cps[dir] = cl;
   p->cc_pair[dir] = pair;
   p->cc_xcd[dir] = xcd;
   p->tune_pending = false;

@@ -28,10 +28,19 @@
 namespace tridhip {
 
 // Largest work-group of k_cc_sweep for chunk length R and NS systems per
-// lane (its launch bound): 64 chunk rows per lane (R = 32 with two systems)
-// need more than the 128 VGPRs of a 1024-thread work-group.
-__host__ __device__ constexpr int cc_max_threads(int R, int NS) {
-  return R * NS >= 64 ? 512 : 1024;
+// lane (its launch bound): 64 FP64 chunk rows per lane (R = 32 with two
+// systems) need more than the 128 VGPRs of a 1024-thread work-group; FP32
+// ones fit (126) with 32-bit offsets.
+__host__ __device__ constexpr int cc_max_threads(int R, int NS, size_t tsize, size_t isize) {
+  return (tsize == 8 || isize == 8) && R * NS >= 64 ? 512 : 1024;
+}
+
+// PCR levels of a reduced system of cps rows (any cps: a neighbour past
+// either end is the zero row).
+__host__ __device__ inline int cc_levels(int cps) {
+  int l = 0;
+  while ((1 << l) < cps) l++;
+  return l;
 }
 
 // Per-chunk factor record (T values) for chunk length R.
@@ -57,16 +66,14 @@ struct CCLayout {
 
 // Factors of the interior-line matrix of a constant-coefficient batch (rows
 // interior to the grid when 1 <= row <= N-2: a, b, c = cf; identity rows
-// otherwise), for chunk length R and cps = 2^cps_log2 chunks.  One
-// wave (cps <= 64); thread k writes chunk k's record at F + k * nf.  The recurrences are those of chunk_reduce, eliminate_first
+// otherwise), for chunk length R and cps chunks.  One
+// wave (cps <= 64; sa and sc: 64 values of LDS each); thread k writes chunk k's record at F + k * nf.  The recurrences are those of chunk_reduce, eliminate_first
 // and pcr_update, applied to the coefficients only.
 template <typename T, int R>
-__global__ void __launch_bounds__(kWave)
-    k_cc_setup(CoefConst<T> cf, int N, int cps_log2, T *__restrict__ F) {
+__device__ __forceinline__ void cc_setup_wave(CoefConst<T> cf, int N, int cps, T *__restrict__ F,
+                                              T *sa, T *sc) {
   using Ly = CCLayout<R>;
-  __shared__ T sa[kWave], sc[kWave];
-  const int cps = 1 << cps_log2;
-  const int nf = Ly::nf(cps_log2);
+  const int nf = Ly::nf(cc_levels(cps));
   const int k = threadIdx.x;
   const bool on = k < cps;
   T *out = F + (long long)(on ? k : 0) * nf;
@@ -153,8 +160,15 @@ __global__ void __launch_bounds__(kWave)
   }
 }
 
+template <typename T, int R>
+__global__ void __launch_bounds__(kWave)
+    k_cc_setup(CoefConst<T> cf, int N, int cps, T *__restrict__ F) {
+  __shared__ T sa[kWave], sc[kWave];
+  cc_setup_wave<T, R>(cf, N, cps, F, sa, sc);
+}
+
 // The solve with precomputed factors F (k_cc_setup of the same N, R, cps).
-// blockDim = 64 * cps <= cc_max_threads(R, NS); wave w = chunk w; lane l of work-group b takes NS
+// blockDim = 64 * cps within the launch bound (any cps); wave w = chunk w; lane l of work-group b takes NS
 // adjacent systems q = NS * (64 * b + l) + s, s < NS.  NS = 2 moves both
 // systems' rows as one 16-byte access (the host requires adjacent systems to
 // be adjacent elements of d and u, 16-byte aligned, and an even system
@@ -162,18 +176,17 @@ __global__ void __launch_bounds__(kWave)
 // Non-Inc: d <- A^{-1} d; Inc: u <- u + A^{-1} d.  CP: cache policy of the
 // streaming accesses (kStream / kCached).
 template <typename T, int INC, int R, typename I, int NS, int CP>
-__global__ void __launch_bounds__(cc_max_threads(R, NS))
+__global__ void __launch_bounds__(cc_max_threads(R, NS, sizeof(T), sizeof(I)))
     k_cc_sweep(const T *__restrict__ F, T *__restrict__ Dd, T *__restrict__ U, SysDesc D,
-               int cps_log2, int xcd) {
+               int cps, int xcd) {
   using Ly = CCLayout<R>;
   typedef T V2 __attribute__((ext_vector_type(2)));
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *sm = reinterpret_cast<T *>(smem_raw);
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
-  const int cps = 1 << cps_log2;
   const int k = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform chunk index
-  const T *__restrict__ Fk = F + k * Ly::nf(cps_log2);
+  const T *__restrict__ Fk = F + k * Ly::nf(cc_levels(cps));
   // xcd: every XCD takes one contiguous range of systems (as k_part)
   long long block = blockIdx.x;
   if (xcd) {
