@@ -37,13 +37,19 @@ __global__ void __launch_bounds__(((R >= 16 && sizeof(T) == 8) || VEC == 4) ? 51
 
 // Segment steps of a split-line solve: D's systems are segments of longer
 // systems.  MODE 1: their merged reduced rows go to `so`; MODE 2: solved
-// with the couplings to the neighbouring segments taken from so.rd.
-template <typename T, int MODE, int INC, int ORDER, int R, int VEC, typename I>
-__global__ void __launch_bounds__((R >= 16 && sizeof(T) == 8) ? 512 : 1024)
+// with the couplings to the neighbouring segments taken from so.rd.  xcd as
+// in k_part.
+template <typename T, int MODE, int INC, int ORDER, int R, int VEC, typename I, int CP>
+__global__ void __launch_bounds__(((R >= 16 && sizeof(T) == 8) || VEC == 4) ? 512 : 1024)
     k_seg(CoefArrays<T> coef, T *__restrict__ Dd, T *__restrict__ U, SysDesc D, int cps_log2,
-          int spb_log2, SegOut<T> so) {
-  part_block<T, INC, ORDER, R, VEC, I, CoefArrays<T>, MODE>(
-      coef, Dd, U, D, cps_log2, spb_log2, blockIdx.x, nullptr, so);
+          int spb_log2, int xcd, SegOut<T> so) {
+  long long block = blockIdx.x;
+  if (xcd) {
+    const unsigned nb8 = gridDim.x & ~7u;
+    if (blockIdx.x < nb8) block = (long long)(blockIdx.x & 7u) * (nb8 >> 3) + (blockIdx.x >> 3);
+  }
+  part_block<T, INC, ORDER, R, VEC, I, CoefArrays<T>, MODE, CP>(
+      coef, Dd, U, D, cps_log2, spb_log2, block, nullptr, so);
 }
 
 struct PartCfg {
@@ -169,12 +175,15 @@ hipError_t launch_seg_t(const PartCfg &cfg, const CoefArrays<T> &coef, T *d, T *
   // unless all chunks of a segment are in one wave (ORDER 0, cps <= 64)
   if (ORDER == 1 || cps > kWave) lds = 2 * 3 * (size_t)cps * (spb + 1) * sizeof(T);
   if (VEC == 2) lds = (size_t)threads * R * sizeof(T);
-  if (cfg.idx32)
-    hipLaunchKernelGGL((k_seg<T, MODE, INC, ORDER, R, VEC, uint32_t>), dim3((unsigned)blocks),
-                       dim3(threads), lds, st, coef, d, u, D, cfg.cps_log2, cfg.spb_log2, so);
-  else
-    hipLaunchKernelGGL((k_seg<T, MODE, INC, ORDER, R, VEC, long long>), dim3((unsigned)blocks),
-                       dim3(threads), lds, st, coef, d, u, D, cfg.cps_log2, cfg.spb_log2, so);
+  if (VEC == 4) lds = (size_t)(threads / kWave) * (kWave * R + 16 / sizeof(T)) * sizeof(T);
+#define TRID_SEG_K(II, CC)                                                                  \
+  hipLaunchKernelGGL((k_seg<T, MODE, INC, ORDER, R, VEC, II, CC>), dim3((unsigned)blocks),  \
+                     dim3(threads), lds, st, coef, d, u, D, cfg.cps_log2, cfg.spb_log2, \
+                     cfg.xcd, so)
+  if (!cfg.idx32) TRID_SEG_K(long long, kStream);
+  else if (cfg.cp == kCached) TRID_SEG_K(uint32_t, kCached);
+  else TRID_SEG_K(uint32_t, kStream);
+#undef TRID_SEG_K
   return hipGetLastError();
 }
 
@@ -195,6 +204,8 @@ hipError_t launch_seg(const PartCfg &cfg, const CoefArrays<T> &coef, T *d, T *u,
   TRID_SEG(0, 4, 2)
   TRID_SEG(0, 8, 2)
   TRID_SEG(0, 16, 2)
+  TRID_SEG(0, 8, 4)
+  TRID_SEG(0, 16, 4)
   TRID_SEG(1, 4, 0)
   TRID_SEG(1, 8, 0)
   TRID_SEG(1, 16, 0)
@@ -438,7 +449,7 @@ inline PartCfg split_cfg(int order, int vec, size_t tsize, long long nsys) {
   c.kind = 4;
   c.order = order;
   c.R = tsize == 8 ? 8 : 16;
-  c.vec = order == 0 && vec && (c.R * (int)tsize) % 16 == 0;
+  c.vec = order == 0 && vec && (c.R * (int)tsize) % 16 == 0;  // (split_vec decides)
   if (order == 0) {
     c.cps_log2 = 6;
     c.spb_log2 = 2;
@@ -448,6 +459,22 @@ inline PartCfg split_cfg(int order, int vec, size_t tsize, long long nsys) {
     if (c.spb_log2 + c.cps_log2 < 6) c.spb_log2 = 6 - c.cps_log2;
   }
   return c;
+}
+
+// Row access of a split-line configuration's segment kernels for systems of
+// N rows: ORDER 0 segments that fill a wave (64 chunks) move as spans, exactly
+// staged where every segment is whole and 16-byte aligned (vec), else through
+// the general staging (gvec: unit stride, 16-byte aligned bases); shorter
+// segments staged only where the segments of a wave are whole and adjacent.
+inline int split_vec(const PartCfg &c, int N, int vec, bool gvec, size_t tsize) {
+  if (c.order != 0) return 0;
+  const int L = c.R << c.cps_log2, cps = 1 << c.cps_log2, P = (N + L - 1) / L;
+  const bool v = vec && (c.R * (int)tsize) % 16 == 0;
+  if (v && N % L == 0 && cps <= kWave && P % (kWave / cps) == 0) return 2;
+  if (gvec && cps == kWave && (c.R == 8 || c.R == 16) &&
+      (1 << (c.cps_log2 + c.spb_log2)) <= 512)
+    return 4;
+  return v;
 }
 
 inline PartCfg heuristic(int order, int N, int vec, size_t tsize) {

@@ -133,36 +133,36 @@ __device__ __forceinline__ void seg_merge(Row<T> &f, Row<T> &l, const Row<T> &fb
   l = L;
 }
 
-// Output of the segment-reduction mode of part_block (split-line solves of
-// systems longer than one work-group holds).  The work-group's systems are
-// segments of L rows of longer systems; each segment's two merged reduced
-// rows go to rows 2p and 2p+1 of its system's reduced system (b = 1), at
-// element qs * rs_sys + row * rs_row of ra, rb, rc, rd.
-//   segment item q -> (system qs, segment p): p_tail >= 0: the launch holds
-//   only the last (partial) segment p_tail of every system, qs = q;
-//   otherwise ORDER 0: p = q % Pf, qs = q / Pf; ORDER 1: qs = q % nsys,
-//   p = q / nsys.
+// Segments of split-line solves (systems longer than one work-group holds):
+// the work-group's systems are segments of L = SysDesc::N rows of longer
+// systems of N rows each, P per system, the last one possibly shorter.  Each
+// segment's two merged reduced rows go to rows 2p and 2p+1 of its system's
+// reduced system of 2P rows (b = 1), at element 2P * qs + row of ra, rb, rc,
+// rd: reduced systems are contiguous whatever the order of the long ones.
+//   segment item q -> (system qs, segment p): ORDER 0: p = q % P, qs = q / P;
+//   ORDER 1: qs = q % nsys, p = q / nsys.
 template <typename T>
 struct SegOut {
   T *ra = nullptr, *rb = nullptr, *rc = nullptr, *rd = nullptr;
-  long long rs_row = 0, rs_sys = 0;
   long long nsys = 0;
-  int Pf = 1, P = 1, p_tail = -1;
+  int P = 1, N = 0;
 };
 
-// (system, segment) of segment item q of a SegOut launch.
+// (system, segment) of segment item q.
 template <typename T, int ORDER>
-__device__ __forceinline__ void seg_item(const SegOut<T> &so, long long q, long long &qs,
-                                         int &p) {
-  if (so.p_tail >= 0) {
-    qs = q;
-    p = so.p_tail;
+__device__ __forceinline__ void seg_item(const SegOut<T> &so, bool small, long long q,
+                                         long long &qs, int &p) {
+  if (small) {
+    const unsigned uq = (unsigned)q, d = ORDER == 0 ? (unsigned)so.P : (unsigned)so.nsys;
+    const unsigned quo = uq / d, rem = uq - quo * d;
+    qs = ORDER == 0 ? quo : rem;
+    p = (int)(ORDER == 0 ? rem : quo);
   } else if (ORDER == 0) {
-    p = (int)(q % so.Pf);
-    qs = q / so.Pf;
+    qs = q / so.P;
+    p = (int)(q - qs * so.P);
   } else {
-    qs = q % so.nsys;
     p = (int)(q / so.nsys);
+    qs = q - (long long)p * so.nsys;
   }
 }
 
@@ -845,7 +845,14 @@ __device__ __forceinline__ void part_block(const Coef &coef, T *__restrict__ Dd,
   }
   const long long q = block * spb + slot;
   const bool active = q < D.nsys;
-  const int N = D.N;
+  long long seg_qs = 0;  // MODE 1, 2: the lane's system and segment
+  int seg_p = 0, rows = D.N;
+  if constexpr (MODE != 0) {
+    if (active) seg_item<T, ORDER>(so, D.small_index, q, seg_qs, seg_p);
+    const long long left = so.N - (long long)seg_p * D.N;
+    rows = left < D.N ? (int)left : D.N;
+  }
+  const int N = rows;
   I off[5];
   bool line_in = false;
   if (active) {
@@ -877,7 +884,7 @@ __device__ __forceinline__ void part_block(const Coef &coef, T *__restrict__ Dd,
     if (cps <= kWave) {
       // whole systems, dense: system q at q * N in every array
       const long long nact = D.nsys - q0 < (kWave >> cps_log2) ? D.nsys - q0 : (kWave >> cps_log2);
-      wave_len = (int)(nact * N);
+      wave_len = (int)(nact * N);  // (segments: one per wave, cps = 64)
       g_idx = (int)(q - q0) * N + row0;
     } else {
       // 64 chunks of one system
@@ -1057,14 +1064,10 @@ __device__ __forceinline__ void part_block(const Coef &coef, T *__restrict__ Dd,
   }
   if constexpr (MODE == 2) {
     if (active && (row0 == 0 || row0 + R == N)) {
-      long long qs;
-      int p;
-      seg_item<T, ORDER>(so, q, qs, p);
-      const long long xb = qs * so.rs_sys;
-      if (row0 == 0 && p > 0)
-        d[0] -= *at(coef.A, off[0]) * so.rd[xb + (2LL * p - 1) * so.rs_row];
-      if (row0 + R == N && p + 1 < so.P)
-        d[R - 1] -= *at(coef.C, off[2] + (I)(N - 1) * s2) * so.rd[xb + (2LL * p + 2) * so.rs_row];
+      const T *x = so.rd + (2LL * so.P * seg_qs + 2LL * seg_p);
+      if (row0 == 0 && seg_p > 0) d[0] -= *at(coef.A, off[0]) * x[-1];
+      if (row0 + R == N && seg_p + 1 < so.P)
+        d[R - 1] -= *at(coef.C, off[2] + (I)(N - 1) * s2) * x[2];
     }
   }
   if constexpr (MODE == 1) {
@@ -1128,21 +1131,17 @@ __device__ __forceinline__ void part_block(const Coef &coef, T *__restrict__ Dd,
       }
     }
     if (k == 0 && active) {
-      long long qs;
-      int p;
-      seg_item<T, ORDER>(so, q, qs, p);
-      const T as = p > 0 ? *at(coef.A, off[0]) : T(0);
-      const T ce = p + 1 < so.P ? *at(coef.C, off[2] + (I)(N - 1) * s2) : T(0);
-      const long long i0 = qs * so.rs_sys + (long long)(2 * p) * so.rs_row;
-      const long long i1 = i0 + so.rs_row;
+      const T as = seg_p > 0 ? *at(coef.A, off[0]) : T(0);
+      const T ce = seg_p + 1 < so.P ? *at(coef.C, off[2] + (I)(N - 1) * s2) : T(0);
+      const long long i0 = 2LL * so.P * seg_qs + 2LL * seg_p;
       so.ra[i0] = f.a * as;
       so.rb[i0] = T(1);
       so.rc[i0] = f.c;
       so.rd[i0] = f.d;
-      so.ra[i1] = l.a;
-      so.rb[i1] = T(1);
-      so.rc[i1] = l.c * ce;
-      so.rd[i1] = l.d;
+      so.ra[i0 + 1] = l.a;
+      so.rb[i0 + 1] = T(1);
+      so.rc[i0 + 1] = l.c * ce;
+      so.rd[i0 + 1] = l.d;
     }
     return;
   }

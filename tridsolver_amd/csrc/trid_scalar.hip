@@ -128,18 +128,78 @@ hipError_t launch_fallback(const T *a, const T *b, const T *c, T *d, T *u,
 // ranks (scalar/src/cpu/trid_mpi_cpu.hpp:139-328: modified Thomas per rank,
 // reduced system of two rows per rank, then a backward pass per rank); here
 // the ranks are segments of one GPU's batch.
+// Bound by the two passes over a, b, c, d: 48 x 150000 rows FP64, solvedim 1:
+// 54 + 13 (reduced systems) + 46 us (the reduced systems in the long systems'
+// own order, one launch of few work-groups: 61 us; tails in launches of their
+// own: 5 us each), 162 -> 111 us in all; 17641 x 9, solvedim 0: 37 -> 23 us.
 
 inline long long round4(long long v) { return (v + 3) & ~3LL; }
 
+// Untuned configuration of a strided batch: the heuristic chunk layout,
+// the strided default for solvedim >= 1, wave staging where it applies and
+// the chunk length that pads a solvedim-0 system least.
+template <typename T>
+PartCfg default_cfg(int order, const SysDesc &D, int vec, bool gvec, bool dense) {
+  PartCfg cfg = heuristic(order, D.N, vec, sizeof(T));
+  if (order == 1 && cfg.kind == 1) {
+    const PartCfg s = strided_default(D.N, sizeof(T));
+    if (s.kind == 1) cfg = s;
+  }
+  // staging pays when a chunk is more than one 16-byte vector
+  if (cfg.R * sizeof(T) > 16) {
+    if (stage_ok(cfg, dense, D.nsys, D.N)) {
+      cfg.vec = staged_vec(cfg);
+    } else {
+      // general staging takes up to 512 threads: longer FP64 chunks if
+      // needed (FP32 is faster unstaged than in 16-row chunks)
+      PartCfg c16 = make_cfg(order, 16, D.N, cfg.vec, 256);
+      if (sizeof(T) == 8 && !gstage_ok(cfg, gvec, dense) && cfg_valid(c16, D.N) &&
+          gstage_ok(c16, gvec, dense))
+        cfg = c16;
+      if (gstage_ok(cfg, gvec, dense)) cfg.vec = 4;
+    }
+  }
+  // solvedim 0 between powers of two: 12-row chunks when they pad less
+  return pick_rows(cfg, D.N, gvec, dense, sizeof(T));
+}
+
+// Configuration of the reduced systems (2P contiguous rows each, ns of them):
+// one launch, or a split-line solve of their own past one work-group.
+template <typename T>
+PartCfg reduced_cfg(const SysDesc &Dr) {
+  const int vec = (Dr.N * (int)sizeof(T)) % 16 == 0;
+  PartCfg c = default_cfg<T>(0, Dr, vec, true, true);
+  if (c.kind != 1) {
+    c = split_cfg(0, vec, sizeof(T), Dr.nsys);
+    c.vec = split_vec(c, Dr.N, vec, true, sizeof(T));
+  }
+  return c;
+}
+
+SysDesc reduced_desc(int P, long long ns) {
+  SysDesc D;
+  memset(&D, 0, sizeof D);
+  D.N = 2 * P;
+  D.nsys = ns;
+  D.nother = 1;
+  D.osize[0] = (int)ns;
+  for (int t = 0; t < 5; t++) {
+    D.sstr[t] = 1;
+    D.ostr[t][0] = 2LL * P;
+  }
+  D.small_index = !wide_index();
+  return D;
+}
+
 // Workspace (elements) of a split-line solve, including its recursive
 // reduced solves.
-inline long long split_ws_elems(const PartCfg &cfg, int N, long long nsys, size_t tsize) {
+template <typename T>
+long long split_ws_elems(const PartCfg &cfg, int N, long long nsys) {
   const long long L = (long long)cfg.R << cfg.cps_log2;
   const long long P = (N + L - 1) / L;
-  const long long n2 = round4(2 * P * nsys);
-  long long need = 4 * n2;
-  if (heuristic(cfg.order, (int)(2 * P), 1, tsize).kind != 1)
-    need += split_ws_elems(split_cfg(cfg.order, 1, tsize, nsys), (int)(2 * P), nsys, tsize);
+  long long need = 4 * round4(2 * P * nsys);
+  const PartCfg cr = reduced_cfg<T>(reduced_desc((int)P, nsys));
+  if (cr.kind != 1) need += split_ws_elems<T>(cr, (int)(2 * P), nsys);
   return need;
 }
 
@@ -148,116 +208,55 @@ hipError_t split_solve(const PartCfg &cfg, const T *a, const T *b, const T *c, T
                        T *u, const SysDesc &D, hipStream_t st, T *ws) {
   const int order = cfg.order;
   const int L = cfg.R << cfg.cps_log2;
-  const int N = D.N;
-  const int P = (N + L - 1) / L, Pf = N / L;
-  const int Nt = N - Pf * L;
+  const int N = D.N, P = (N + L - 1) / L;
   const long long ns = D.nsys;
   const long long n2 = round4(2LL * P * ns);
-  T *ra = ws, *rb = ws + n2, *rc = ws + 2 * n2, *rd = ws + 3 * n2;
-  T *next = ws + 4 * n2;
 
   SegOut<T> so;
-  so.ra = ra;
-  so.rb = rb;
-  so.rc = rc;
-  so.rd = rd;
+  so.ra = ws;
+  so.rb = ws + n2;
+  so.rc = ws + 2 * n2;
+  so.rd = ws + 3 * n2;
   so.nsys = ns;
   so.P = P;
-  so.Pf = Pf > 0 ? Pf : 1;
-  so.rs_row = order == 0 ? 1 : ns;
-  so.rs_sys = order == 0 ? 2LL * P : 1;
+  so.N = N;
 
-  // the full segments as one batch: the segment index is one more non-solve
+  // the segments as one batch: the segment index is one more non-solve
   // dimension (fastest for ORDER 0, so that a system's segments are adjacent
   // work items; slowest for ORDER 1, which keeps systems in adjacent lanes)
   SysDesc Ds = D;
   Ds.N = L;
-  if (Pf > 0) {
-    const int slot = order == 0 ? 0 : D.nother;
-    for (int k = D.nother; k > slot; k--) {
-      Ds.osize[k] = D.osize[k - 1];
-      for (int t = 0; t < 5; t++) Ds.ostr[t][k] = D.ostr[t][k - 1];
-    }
-    Ds.osize[slot] = Pf;
-    for (int t = 0; t < 5; t++) Ds.ostr[t][slot] = (long long)L * D.sstr[t];
-    Ds.nother = D.nother + 1;
-    Ds.nsys = ns * Pf;
-    Ds.small_index = Ds.nsys < (1LL << 31) && !wide_index();
+  const int slot = order == 0 ? 0 : D.nother;
+  for (int k = D.nother; k > slot; k--) {
+    Ds.osize[k] = D.osize[k - 1];
+    for (int t = 0; t < 5; t++) Ds.ostr[t][k] = D.ostr[t][k - 1];
   }
+  Ds.osize[slot] = P;
+  for (int t = 0; t < 5; t++) Ds.ostr[t][slot] = (long long)L * D.sstr[t];
+  Ds.nother = D.nother + 1;
+  Ds.nsys = ns * P;
+  Ds.small_index = Ds.nsys < (1LL << 31) && !wide_index();
   PartCfg cs = cfg;
   cs.kind = 1;
-  cs.xcd = 0;
-  if (cs.vec == 2) cs.vec = 1;
-  // wave-staged access: the segments of one wave must be adjacent in memory
-  if (cs.vec == 1 && order == 0 && (1 << cs.cps_log2) <= kWave &&
-      Pf % (kWave >> cs.cps_log2) == 0)
-    cs.vec = 2;
 
-  // the last, shorter segment of every system (rows Pf*L .. N-1)
-  SysDesc Dt = D;
-  Dt.N = Nt;
-  PartCfg ct;
-  const long long sh[5] = {(long long)Pf * L * D.sstr[0], (long long)Pf * L * D.sstr[1],
-                           (long long)Pf * L * D.sstr[2], (long long)Pf * L * D.sstr[3],
-                           (long long)Pf * L * D.sstr[4]};
-  if (Nt > 0) {
-    ct = make_cfg(order, cfg.R, Nt, cfg.vec ? 1 : 0, 1 << (cfg.cps_log2 + cfg.spb_log2));
-    ct.idx32 = cfg.idx32;
-    if (!cfg_valid(ct, Nt)) return hipErrorInvalidValue;
-  }
-
-  SegOut<T> sot = so;  // the tail launch
-  sot.p_tail = Pf;
-
-  hipError_t e;
+  const CoefArrays<T> cf{a, b, c};
   // 1. segment reduction
-  if (Pf > 0) {
-    e = launch_seg<T, 1, 0>(cs, CoefArrays<T>{a, b, c}, d, nullptr, Ds, so, st);
-    if (e != hipSuccess) return e;
-  }
-  if (Nt > 0) {
-    e = launch_seg<T, 1, 0>(ct, CoefArrays<T>{a + sh[0], b + sh[1], c + sh[2]}, d + sh[3],
-                            nullptr, Dt, sot, st);
-    if (e != hipSuccess) return e;
-  }
+  hipError_t e = launch_seg<T, 1, 0>(cs, cf, d, nullptr, Ds, so, st);
+  if (e != hipSuccess) return e;
 
-  // 2. reduced systems: 2P rows each, laid out like the original order
-  SysDesc Dr;
-  memset(&Dr, 0, sizeof Dr);
-  Dr.N = 2 * P;
-  Dr.nsys = ns;
-  Dr.nother = 1;
-  Dr.osize[0] = (int)ns;
-  for (int t = 0; t < 5; t++) {
-    Dr.sstr[t] = so.rs_row;
-    Dr.ostr[t][0] = so.rs_sys;
-  }
-  Dr.small_index = !wide_index();
-  const int ridx32 = (unsigned long long)n2 * sizeof(T) < (1ULL << 32) && !wide_index();
-  // (16-byte loads along the reduced rows for ORDER 0: the workspace arrays
-  // are 16-byte aligned and each system's 2P rows start at a multiple of 2P)
-  const int rvec = order == 0 && (2 * P * (int)sizeof(T)) % 16 == 0;
-  PartCfg cr = heuristic(order, 2 * P, rvec, sizeof(T));
-  if (cr.kind == 1) {
-    if (stage_ok(cr, order == 0, ns, 2 * P)) cr.vec = staged_vec(cr);
-    cr.idx32 = ridx32;
-    e = launch_part<T, 0>(cr, CoefArrays<T>{ra, rb, rc}, rd, nullptr, Dr, st);
-  } else {
-    cr = split_cfg(order, rvec, sizeof(T), ns);
-    cr.idx32 = ridx32;
-    e = split_solve<T, 0>(cr, ra, rb, rc, rd, nullptr, Dr, st, next);
-  }
+  // 2. reduced systems
+  const SysDesc Dr = reduced_desc(P, ns);
+  PartCfg cr = reduced_cfg<T>(Dr);
+  cr.idx32 = (unsigned long long)n2 * sizeof(T) < (1ULL << 32) && !wide_index();
+  cr.cp = cr.idx32 ? kCached : kStream;
+  if (cr.kind == 1)
+    e = launch_part<T, 0>(cr, CoefArrays<T>{so.ra, so.rb, so.rc}, so.rd, nullptr, Dr, st);
+  else
+    e = split_solve<T, 0>(cr, so.ra, so.rb, so.rc, so.rd, nullptr, Dr, st, ws + 4 * n2);
   if (e != hipSuccess) return e;
 
   // 3. independent segments, couplings from the reduced solution
-  if (Pf > 0) {
-    e = launch_seg<T, 2, INC>(cs, CoefArrays<T>{a, b, c}, d, u, Ds, so, st);
-    if (e != hipSuccess) return e;
-  }
-  if (Nt > 0)
-    e = launch_seg<T, 2, INC>(ct, CoefArrays<T>{a + sh[0], b + sh[1], c + sh[2]}, d + sh[3],
-                              INC ? u + sh[4] : nullptr, Dt, sot, st);
-  return e;
+  return launch_seg<T, 2, INC>(cs, cf, d, u, Ds, so, st);
 }
 
 std::mutex g_tune_mu;
@@ -288,7 +287,7 @@ tridStatus_t run_cfg(const PartCfg &cfg, const T *a, const T *b, const T *c,
   if (cfg.kind == 2 || cfg.kind == 4) {
     const size_t bytes =
         cfg.kind == 2 ? 2 * (size_t)D.N * (size_t)D.nsys * sizeof(T)
-                      : (size_t)split_ws_elems(cfg, D.N, D.nsys, sizeof(T)) * sizeof(T);
+                      : (size_t)split_ws_elems<T>(cfg, D.N, D.nsys) * sizeof(T);
     T *ws;
     if (fixed) {
       if (bytes > fixed_bytes)
@@ -370,34 +369,6 @@ PartCfg autotune(int order, int vec, bool gvec, int idx32, bool dense, const T *
   }
   (void)hipMemcpyAsync(dst, saved, bytes, hipMemcpyDeviceToDevice, st);
   return best;
-}
-
-// Untuned configuration of a strided batch: the heuristic chunk layout,
-// the strided default for solvedim >= 1, wave staging where it applies and
-// the chunk length that pads a solvedim-0 system least.
-template <typename T>
-PartCfg default_cfg(int order, const SysDesc &D, int vec, bool gvec, bool dense) {
-  PartCfg cfg = heuristic(order, D.N, vec, sizeof(T));
-  if (order == 1 && cfg.kind == 1) {
-    const PartCfg s = strided_default(D.N, sizeof(T));
-    if (s.kind == 1) cfg = s;
-  }
-  // staging pays when a chunk is more than one 16-byte vector
-  if (cfg.R * sizeof(T) > 16) {
-    if (stage_ok(cfg, dense, D.nsys, D.N)) {
-      cfg.vec = staged_vec(cfg);
-    } else {
-      // general staging takes up to 512 threads: longer FP64 chunks if
-      // needed (FP32 is faster unstaged than in 16-row chunks)
-      PartCfg c16 = make_cfg(order, 16, D.N, cfg.vec, 256);
-      if (sizeof(T) == 8 && !gstage_ok(cfg, gvec, dense) && cfg_valid(c16, D.N) &&
-          gstage_ok(c16, gvec, dense))
-        cfg = c16;
-      if (gstage_ok(cfg, gvec, dense)) cfg.vec = 4;
-    }
-  }
-  // solvedim 0 between powers of two: 12-row chunks when they pad less
-  return pick_rows(cfg, D.N, gvec, dense, sizeof(T));
 }
 
 template <typename T, int INC>
@@ -501,7 +472,6 @@ tridStatus_t solve(const T *a, const int *a_pads, const T *b,
       if (order == 1) cfg.spb_log2 = std::min(cfg.spb_log2, 6);
     }
     if (fc.spb) cfg.spb_log2 = ilog2(fc.spb);
-    cfg.vec = vec && (cfg.R * (int)sizeof(T)) % 16 == 0;
     if (!cfg_valid(cfg, D.N))
       return fail(TRID_STATUS_INVALID_VALUE, "forced configuration does not fit this shape");
   } else if (fc.kind == 1 || fc.kind == 3) {
@@ -565,12 +535,23 @@ tridStatus_t solve(const T *a, const int *a_pads, const T *b,
   if (cfg.kind == 4 && fc.kind != 4) cfg = split_cfg(order, vec, sizeof(T), D.nsys);
   if (cfg.kind == 4 && D.nsys > (1LL << 30))
     return fail(TRID_STATUS_INVALID_VALUE, "split-line solve: too many systems");
+  if (cfg.kind == 4) {
+    cfg.vec = split_vec(cfg, D.N, vec, gvec, sizeof(T));
+    // strided row runs end inside cache lines that the next work-group's
+    // begin in: neighbours share an XCD's L2 ([300, 3000, 10] FP32, ordinary
+    // loads: 95 -> 79 us); whole spans (ORDER 0) share none
+    cfg.xcd = order == 1;
+  }
   cfg.idx32 = idx32;
   // cache policy: the tuned one, else the footprint rule; a forced policy
-  // wins; split-line, fallback and 64-bit-offset solves always stream
+  // wins; fallback and 64-bit-offset solves always stream
   if (!tuned) cfg.cp = cp_rule;
   if (forced_cache_policy() >= 0) cfg.cp = forced_cache_policy();
-  if (!idx32 || cfg.kind != 1) cfg.cp = kStream;
+  if (!idx32 || cfg.kind == 2) cfg.cp = kStream;
+  // split-line: no mixed form, and ORDER 0 streams (2 x 2^22 rows FP64 122
+  // against 132 us with ordinary loads; ORDER 1 [51, 7548, 19] FP32 103
+  // against 77)
+  if (cfg.kind == 4 && (cfg.cp != kCached || order == 0)) cfg.cp = kStream;
   set_last_config(cfg_name(cfg, sizeof(T)));
   // launch events (tridSetLaunchEvents) time single-kernel solves only
   if (cfg.kind != 1) (void)take_launch_events();
