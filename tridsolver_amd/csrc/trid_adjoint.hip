@@ -42,7 +42,7 @@ template <typename T, int ORDER, int R, int VEC, typename I, int CP>
 __global__ void __launch_bounds__((VEC == 4 || (R >= 16 && sizeof(T) == 8)) ? 512 : 1024)
     k_adj(const T *__restrict__ A, const T *__restrict__ B, const T *__restrict__ C,
           const T *__restrict__ X, const T *__restrict__ G, T *__restrict__ GA,
-          T *__restrict__ GB, T *__restrict__ GC, T *__restrict__ GD, SysDesc D, int cps_log2,
+          T *__restrict__ GB, T *__restrict__ GC, T *__restrict__ GD, SysDesc D, int chunks,
           int spb_log2, int xcd) {
   constexpr bool GSTAGE = VEC == 4;
   constexpr int SW = kWave * R + (GSTAGE ? Vec16<T>::n : 0);  // a wave's staging buffer
@@ -54,7 +54,8 @@ __global__ void __launch_bounds__((VEC == 4 || (R >= 16 && sizeof(T) == 8)) ? 51
     if (blockIdx.x < nb8) block = (long long)(blockIdx.x & 7u) * (nb8 >> 3) + (blockIdx.x >> 3);
   }
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
-  const int cps = 1 << cps_log2, spb = 1 << spb_log2;
+  const int cps_log2 = chunks;  // (ORDER 0; ORDER 1: the count, any number)
+  const int cps = ORDER == 0 ? 1 << chunks : chunks, spb = 1 << spb_log2;
   const int k = ORDER == 0 ? tid & (cps - 1) : tid >> spb_log2;
   const int slot = ORDER == 0 ? tid >> cps_log2 : tid & (spb - 1);
   const long long q = block * spb + slot;
@@ -200,7 +201,7 @@ template <typename T, int ORDER, int R, int VEC>
 hipError_t launch_adj_t(const PartCfg &cfg, const T *a, const T *b, const T *c, const T *x,
                         const T *g, T *ga, T *gb, T *gc, T *gd, const SysDesc &D,
                         hipStream_t st) {
-  const int cps = 1 << cfg.cps_log2, spb = 1 << cfg.spb_log2, threads = cps * spb;
+  const int cps = chunk_count(cfg), spb = 1 << cfg.spb_log2, threads = cps * spb;
   const unsigned blocks = (unsigned)((D.nsys + spb - 1) / spb);
   size_t lds = 0;
   if (ORDER == 1 || cps > kWave) lds = 2 * 3 * (size_t)cps * (spb + 1) * sizeof(T);
@@ -209,7 +210,7 @@ hipError_t launch_adj_t(const PartCfg &cfg, const T *a, const T *b, const T *c, 
           sizeof(T);
 #define TRID_ADJ(II, CC)                                                                     \
   hipLaunchKernelGGL((k_adj<T, ORDER, R, VEC, II, CC>), dim3(blocks), dim3(threads), lds, st, a, \
-                     b, c, x, g, ga, gb, gc, gd, D, cfg.cps_log2, cfg.spb_log2, cfg.xcd)
+                     b, c, x, g, ga, gb, gc, gd, D, chunk_arg(cfg), cfg.spb_log2, cfg.xcd)
   if (!cfg.idx32) TRID_ADJ(long long, kStream);
   else if (cfg.cp == kCached) TRID_ADJ(uint32_t, kCached);
   else TRID_ADJ(uint32_t, kStream);
@@ -308,6 +309,8 @@ tridStatus_t strided_adjoint(const T *a, const T *b, const T *c, const T *x, con
     // the strided batches' layout (most systems per work-group)
     const PartCfg s = strided_default(D.N, sizeof(T));
     if (s.kind == 1) cfg = s;
+    const PartCfg w = strided_wide(D.N, D.nsys, sizeof(T));
+    if (w.kind == 1) cfg = w;
   } else {
     const PartCfg s = adj_rows(D.N, aligned, dense);
     if (s.kind == 1) cfg = s;

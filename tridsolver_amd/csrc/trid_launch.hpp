@@ -20,7 +20,8 @@ template <typename T, int INC, int ORDER, int R, int VEC, typename I,
           typename Coef, int CP>
 __global__ void __launch_bounds__(((R >= 16 && sizeof(T) == 8) || VEC == 4) ? 512 : 1024)
     k_part(Coef coef, T *__restrict__ Dd, T *__restrict__ U, SysDesc D,
-           int cps_log2, int spb_log2, int xcd, T *__restrict__ Out) {
+           int chunks, int spb_log2, int xcd, T *__restrict__ Out) {
+  // chunks: log2 of the chunk count (ORDER 0) or the count (ORDER 1)
   // CP: cache policy of the streaming accesses (kStream / kCached)
   // xcd: consecutive hardware blocks go round-robin to the 8 XCDs (each with
   // its own L2); this remap hands every XCD one contiguous range of systems
@@ -31,8 +32,8 @@ __global__ void __launch_bounds__(((R >= 16 && sizeof(T) == 8) || VEC == 4) ? 51
     const unsigned nb8 = gridDim.x & ~7u;
     if (blockIdx.x < nb8) block = (long long)(blockIdx.x & 7u) * (nb8 >> 3) + (blockIdx.x >> 3);
   }
-  part_block<T, INC, ORDER, R, VEC, I, Coef, 0, CP>(coef, Dd, U, D, cps_log2, spb_log2,
-                                                    block, Out);
+  part_block<T, INC, ORDER, R, VEC, I, Coef, 0, CP>(coef, Dd, U, D, chunks, spb_log2, block,
+                                                    Out);
 }
 
 // Segment steps of a split-line solve: D's systems are segments of longer
@@ -41,7 +42,7 @@ __global__ void __launch_bounds__(((R >= 16 && sizeof(T) == 8) || VEC == 4) ? 51
 // in k_part.
 template <typename T, int MODE, int INC, int ORDER, int R, int VEC, typename I, int CP>
 __global__ void __launch_bounds__(((R >= 16 && sizeof(T) == 8) || VEC == 4) ? 512 : 1024)
-    k_seg(CoefArrays<T> coef, T *__restrict__ Dd, T *__restrict__ U, SysDesc D, int cps_log2,
+    k_seg(CoefArrays<T> coef, T *__restrict__ Dd, T *__restrict__ U, SysDesc D, int chunks,
           int spb_log2, int xcd, SegOut<T> so) {
   long long block = blockIdx.x;
   if (xcd) {
@@ -49,13 +50,14 @@ __global__ void __launch_bounds__(((R >= 16 && sizeof(T) == 8) || VEC == 4) ? 51
     if (blockIdx.x < nb8) block = (long long)(blockIdx.x & 7u) * (nb8 >> 3) + (blockIdx.x >> 3);
   }
   part_block<T, INC, ORDER, R, VEC, I, CoefArrays<T>, MODE, CP>(
-      coef, Dd, U, D, cps_log2, spb_log2, block, nullptr, so);
+      coef, Dd, U, D, chunks, spb_log2, block, nullptr, so);
 }
 
 struct PartCfg {
   int kind = 1;  // 1 partitioned, 2 fallback, 4 split-line (segments of R*cps rows)
   int R = 8;
   int cps_log2 = 0;
+  int cps_any = 0;  // ORDER 1: chunk count between the powers of two (0: 1 << cps_log2)
   int spb_log2 = 0;
   int order = 0;
   int vec = 0;
@@ -63,6 +65,12 @@ struct PartCfg {
   int xcd = 0;    // XCD-contiguous block order (see k_part)
   int cp = 0;     // cache policy of the streaming accesses: kStream / kCached / kMixed
 };
+
+// Chunks per system.
+inline int chunk_count(const PartCfg &c) { return c.cps_any ? c.cps_any : 1 << c.cps_log2; }
+
+// The `chunks` argument of part_block.
+inline int chunk_arg(const PartCfg &c) { return c.order == 0 ? c.cps_log2 : chunk_count(c); }
 
 inline bool aligned16(const void *p) {
   return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
@@ -77,7 +85,7 @@ inline int ilog2(long long v) {
 template <typename T, int INC, int ORDER, int R, int VEC, typename Coef>
 hipError_t launch_part_t(const PartCfg &cfg, const Coef &coef, T *d, T *u,
                          const SysDesc &D, hipStream_t st, T *out) {
-  const int cps = 1 << cfg.cps_log2, spb = 1 << cfg.spb_log2;
+  const int cps = chunk_count(cfg), spb = 1 << cfg.spb_log2;
   const int threads = cps * spb;
   const long long blocks = (D.nsys + spb - 1) / spb;
   size_t lds = 0;
@@ -97,20 +105,20 @@ hipError_t launch_part_t(const PartCfg &cfg, const Coef &coef, T *d, T *u,
   if (cfg.idx32 && cfg.cp == kCached)
     return launch_kernel(k_part<T, INC, ORDER, R, VEC, uint32_t, Coef, kCached>,
                          dim3((unsigned)blocks), dim3(threads), (std::uint32_t)lds, st, coef, d,
-                         u, D, cfg.cps_log2, cfg.spb_log2, cfg.xcd, out);
+                         u, D, chunk_arg(cfg), cfg.spb_log2, cfg.xcd, out);
   if constexpr (Coef::kArrays) {
     if (cfg.idx32 && cfg.cp == kMixed)
       return launch_kernel(k_part<T, INC, ORDER, R, VEC, uint32_t, Coef, kMixed>,
                            dim3((unsigned)blocks), dim3(threads), (std::uint32_t)lds, st, coef,
-                           d, u, D, cfg.cps_log2, cfg.spb_log2, cfg.xcd, out);
+                           d, u, D, chunk_arg(cfg), cfg.spb_log2, cfg.xcd, out);
   }
   if (cfg.idx32)
     return launch_kernel(k_part<T, INC, ORDER, R, VEC, uint32_t, Coef, kStream>,
                          dim3((unsigned)blocks), dim3(threads), (std::uint32_t)lds, st, coef, d,
-                         u, D, cfg.cps_log2, cfg.spb_log2, cfg.xcd, out);
+                         u, D, chunk_arg(cfg), cfg.spb_log2, cfg.xcd, out);
   return launch_kernel(k_part<T, INC, ORDER, R, VEC, long long, Coef, kStream>,
                        dim3((unsigned)blocks), dim3(threads), (std::uint32_t)lds, st, coef, d, u,
-                       D, cfg.cps_log2, cfg.spb_log2, cfg.xcd, out);
+                       D, chunk_arg(cfg), cfg.spb_log2, cfg.xcd, out);
 }
 
 // Launches the partitioned kernel for any configuration of the table.
@@ -178,7 +186,7 @@ hipError_t launch_seg_t(const PartCfg &cfg, const CoefArrays<T> &coef, T *d, T *
   if (VEC == 4) lds = (size_t)(threads / kWave) * (kWave * R + 16 / sizeof(T)) * sizeof(T);
 #define TRID_SEG_K(II, CC)                                                                  \
   hipLaunchKernelGGL((k_seg<T, MODE, INC, ORDER, R, VEC, II, CC>), dim3((unsigned)blocks),  \
-                     dim3(threads), lds, st, coef, d, u, D, cfg.cps_log2, cfg.spb_log2, \
+                     dim3(threads), lds, st, coef, d, u, D, chunk_arg(cfg), cfg.spb_log2, \
                      cfg.xcd, so)
   if (!cfg.idx32) TRID_SEG_K(long long, kStream);
   else if (cfg.cp == kCached) TRID_SEG_K(uint32_t, kCached);
@@ -233,9 +241,10 @@ inline bool cfg_valid(const PartCfg &cfg, int N, size_t tsize = 8) {
   if (cfg.R != 4 && cfg.R != 8 && cfg.R != 16 &&
       !(is_fill_rows(cfg.R) && cfg.vec == 4 && cfg.order == 0))
     return false;
-  const long long cps = 1LL << cfg.cps_log2, spb = 1LL << cfg.spb_log2;
+  const long long cps = chunk_count(cfg), spb = 1LL << cfg.spb_log2;
   const long long thr = cps * spb;
-  if (thr < kWave || thr > 1024) return false;
+  if (thr < kWave || thr > 1024 || thr % kWave) return false;
+  if (cfg.cps_any && cfg.order == 0) return false;
   const bool r16_wide = tsize == 4 && cfg.order == 1 && cfg.vec == 0;
   if (cfg.R >= 16 && thr > 512 && !r16_wide) return false;  // register budget of R=16
   if (cfg.vec == 4 && thr > 512) return false;  // launch bound of general staging
@@ -293,7 +302,7 @@ inline std::string cfg_name(const PartCfg &c, size_t tsize) {
              1 << c.spb_log2, c.vec >= 2 ? ",staged" : (c.vec ? ",vec" : ""));
   } else {
     snprintf(buf, sizeof buf, "part<%s,o%d,R%d,cps%d,spb%d%s%s%s>",
-             tsize == 8 ? "double" : "float", c.order, c.R, 1 << c.cps_log2,
+             tsize == 8 ? "double" : "float", c.order, c.R, chunk_count(c),
              1 << c.spb_log2,
              c.vec == 4 ? ",gstaged" : (c.vec >= 2 ? ",staged" : (c.vec ? ",vec" : "")),
              c.xcd ? ",xcd" : "",
@@ -302,6 +311,8 @@ inline std::string cfg_name(const PartCfg &c, size_t tsize) {
   return buf;
 }
 
+inline PartCfg strided_wide(int N, long long nsys, size_t tsize);
+
 inline std::vector<PartCfg> candidates(int order, int N, int vec, size_t tsize,
                                 bool dense, long long nsys, bool gvec = false) {
   std::vector<PartCfg> out;
@@ -309,8 +320,8 @@ inline std::vector<PartCfg> candidates(int order, int N, int vec, size_t tsize,
   const int thr[3] = {256, 512, 1024};
   auto add = [&](const PartCfg &c) {
     for (auto &o : out)
-      if (o.R == c.R && o.cps_log2 == c.cps_log2 && o.spb_log2 == c.spb_log2 &&
-          o.vec == c.vec && o.xcd == c.xcd)
+      if (o.R == c.R && o.cps_log2 == c.cps_log2 && o.cps_any == c.cps_any &&
+          o.spb_log2 == c.spb_log2 && o.vec == c.vec && o.xcd == c.xcd)
         return;
     out.push_back(c);
   };
@@ -335,6 +346,10 @@ inline std::vector<PartCfg> candidates(int order, int N, int vec, size_t tsize,
         add_both(c);
       }
     }
+  if (order == 1) {
+    const PartCfg w = strided_wide(N, nsys, tsize);
+    if (w.kind == 1) add(w);
+  }
   for (int R : {5, 6, 7, 12})
     for (int t : thr) {
       PartCfg c = make_cfg(order, R, N, 0, t);
@@ -362,6 +377,58 @@ inline PartCfg strided_default(int N, size_t tsize) {
   PartCfg t = make_cfg(1, R, N, 0, tsize == 8 ? 512 : 1024);
   t.xcd = N > (tsize == 8 ? 512 : 128);
   if (!cfg_valid(t, N, tsize)) return c;
+  return t;
+}
+
+// Layout of strided batches of at least 64 work-groups, where all of the chip
+// is at work (smaller ones keep strided_default or the heuristic):
+//   * the XCD-contiguous order at every length: a work-group's row runs end
+//     inside cache lines that its neighbours' begin in, and neighbours then
+//     share an L2.  Runs of whole lines lose nothing ([256, 256, 256] FP64
+//     115 -> 112 us, [256, 128, 300] FP32 44.5 -> 45), others gain
+//     ([149, 100, 300] FP32 27 -> 19, [149, 220, 244] FP64 91 -> 71).
+//   * the chunk count cut to the rows where that drops a quarter of the
+//     power of two or more (150 rows: 20 chunks of 8, not 32), which makes
+//     room for twice the systems side by side ([150, 150, 150] FP64 35 -> 32
+//     us, [300, 333, 150] FP32 81 -> 74); nearer the power of two the extra
+//     idle lanes cost nothing (220 rows: 28 chunks 77, 32 chunks 71 us).
+//   * FP64, 257..512 rows: 8 systems in 256 threads, four work-groups per CU,
+//     against 16 in 512 ([149, 450, 119] 89 -> 80 us); 513..768 rows: 8-row
+//     chunks, which leave fewer rows idle ([256, 600, 52] 95 -> 79 us).
+//   * FP32 up to 128 rows: 16-row chunks ([149, 128, 300] 26.7 -> 26.3 us,
+//     [256, 70, 300] 25 -> 22); 385..512 rows: 16 systems in 512 threads
+//     ([149, 450, 178] 71 -> 68).
+// Microseconds on MI355X, batches cycled through several sets of arrays.
+// Returns kind 0 when the rule does not apply.
+inline PartCfg strided_wide(int N, long long nsys, size_t tsize) {
+  PartCfg c;
+  c.kind = 0;
+  if (N > 2048) return c;
+  int R, spb;
+  if (tsize == 8) {
+    R = N <= 256 || (N > 512 && N <= 768) ? 8 : 16;
+    spb = N <= 256 ? 512 / std::max(8, 1 << ilog2((N + 7) / 8)) : N <= 1024 ? 8 : 4;
+  } else {
+    R = N > 128 && N <= 256 ? 8 : 16;
+    spb = N <= 128 ? 64 : N <= 384 ? 32 : N <= 1024 ? 16 : 8;
+  }
+  const int chunks = (N + R - 1) / R, cps = 1 << ilog2(chunks);
+  PartCfg t = make_cfg(1, R, N, 0, 512);
+  t.spb_log2 = ilog2(spb);
+  if (t.spb_log2 + t.cps_log2 < 6) return c;  // less than a wave
+  // whole waves: chunks * spb a multiple of 64
+  auto trim = [&](int side) {
+    const int m = side >= kWave ? 1 : kWave / side;
+    return (chunks + m - 1) / m * m;
+  };
+  if (tsize == 8 && N <= 256 && cps >= 16 && 4 * trim(32) <= 3 * cps) {
+    t.spb_log2 = 5;
+    t.cps_any = trim(32);
+  } else if (4 * trim(spb) <= 3 * cps && (tsize == 4 ? N > 128 : N > 512 && N <= 768)) {
+    t.cps_any = trim(spb);
+  }
+  t.xcd = 1;
+  if (!cfg_valid(t, N, tsize) || (nsys >> t.spb_log2) < 64) return c;
   return t;
 }
 

@@ -183,7 +183,7 @@ __device__ __forceinline__ Row<T> row_from_lane(const Row<T> &v, int src,
 }
 
 // Reduced solve for a system whose cps chunks sit in consecutive lanes of
-// one wave (cps a power of two <= 64).  k: the lane's chunk index.
+// one wave (cps <= 64).  k: the lane's chunk index.
 // Returns the chunk's first (xf) and last (xl) unknowns.
 template <typename T>
 __device__ __forceinline__ void reduced_wave(const Row<T> &f, const Row<T> &l,
@@ -252,15 +252,16 @@ __device__ __forceinline__ void reduced_lds(const Row<T> &f, const Row<T> &l,
   }
 }
 
-// Same, for chunks spread over several waves with cps <= 64: the chunks'
-// two reduced rows go to LDS, every wave then takes whole systems (64 / cps
-// systems, chunks in consecutive lanes) and solves them with the in-wave
-// PCR of reduced_wave (no barrier per level), and the chunks' unknowns go
-// back through LDS -- three barriers in all instead of one per PCR level.
-// Entry (chunk k, system slot s) lives at k * (spb + 1) + s of six arrays of
-// cps * (spb + 1) values (the padding keeps the wave-local reads, which walk
-// k with s fixed, free of bank conflicts).  All threads call it; blockDim =
-// cps * spb.
+// Same, for chunks spread over several waves with cps <= 64 (any count): the
+// chunks' two reduced rows go to LDS, every wave then takes whole systems
+// (64 / cps systems at a time, chunks in consecutive lanes) and solves them
+// with the in-wave PCR of reduced_wave (no barrier per level), and the
+// chunks' unknowns go back through LDS -- two barriers in all instead of one
+// per PCR level.  Entry (chunk k, system slot s) lives at k * (spb + 1) + s of
+// six arrays of cps * (spb + 1) values (the padding keeps the wave-local
+// reads, which walk k with s fixed, free of bank conflicts); between the
+// barriers only the one lane that solves for it touches an entry.  All
+// threads call it; blockDim = cps * spb, whole waves.
 template <typename T>
 __device__ __forceinline__ void reduced_lds_w(const Row<T> &f, const Row<T> &l, int k, int cps,
                                               int slot, int spb, T *sm, T &xf, T &xl) {
@@ -275,17 +276,21 @@ __device__ __forceinline__ void reduced_lds_w(const Row<T> &f, const Row<T> &l, 
   sm[5 * n + me] = l.d;
   __syncthreads();
   const int lane = threadIdx.x & (kWave - 1);
-  const int cps_log2 = __builtin_ctz(cps);
-  const int k2 = lane & (cps - 1);
-  const int s2 = (int)(threadIdx.x >> 6) * (kWave >> cps_log2) + (lane >> cps_log2);
-  const int e = k2 * sp + s2;
-  const Row<T> f2{sm[e], sm[n + e], sm[2 * n + e]};
-  const Row<T> l2{sm[3 * n + e], sm[4 * n + e], sm[5 * n + e]};
-  T xf2, xl2;
-  reduced_wave<T>(f2, l2, k2, cps, lane, xf2, xl2);
-  __syncthreads();  // every entry has been read
-  sm[e] = xf2;
-  sm[n + e] = xl2;
+  const int per = kWave / cps;  // systems per wave and turn
+  const int s1 = lane / cps, k2 = lane - s1 * cps;
+  const int step = (int)(blockDim.x >> 6) * per;
+  for (int s0 = (int)(threadIdx.x >> 6) * per; s0 < spb; s0 += step) {
+    const bool on = s1 < per && s0 + s1 < spb;
+    const int e = on ? k2 * sp + s0 + s1 : 0;
+    const Row<T> f2{sm[e], sm[n + e], sm[2 * n + e]};
+    const Row<T> l2{sm[3 * n + e], sm[4 * n + e], sm[5 * n + e]};
+    T xf2, xl2;
+    reduced_wave<T>(f2, l2, k2, cps, lane, xf2, xl2);
+    if (on) {
+      sm[e] = xf2;
+      sm[n + e] = xl2;
+    }
+  }
   __syncthreads();
   xf = sm[me];
   xl = sm[n + me];
@@ -802,8 +807,9 @@ struct CoefKappa {
 //            wave a contiguous span of one system), with the wave-blocked
 //            reduced solve (reduced_multi).
 //   I:       index type of element offsets (uint32_t or long long).
-// blockDim.x == cps * spb, both powers of two.  Non-Inc: d <- A^{-1} d;
-// Inc: u <- u + A^{-1} d.
+// blockDim.x == cps * spb, whole waves.  ORDER 0 and MODE 1: powers of two,
+// `chunks` is log2 of cps; ORDER 1 (MODE 0 and 2): `chunks` is cps, any count.
+// Non-Inc: d <- A^{-1} d; Inc: u <- u + A^{-1} d.
 // MODE 1 (segment reduction, CoefArrays only): every system of D is a
 // segment of a longer system; instead of solving it, the work-group merges
 // each segment's chunk rows into the segment's two reduced rows -- with the
@@ -818,7 +824,7 @@ template <typename T, int INC, int ORDER, int R, int VEC, typename I,
           typename Coef, int MODE = 0, int CP = kStream>
 __device__ __forceinline__ void part_block(const Coef &coef, T *__restrict__ Dd,
                                            T *__restrict__ U, const SysDesc &D,
-                                           int cps_log2, int spb_log2,
+                                           int chunks, int spb_log2,
                                            long long block,
                                            T *__restrict__ Out = nullptr,
                                            SegOut<T> so = SegOut<T>()) {
@@ -833,7 +839,8 @@ __device__ __forceinline__ void part_block(const Coef &coef, T *__restrict__ Dd,
   // per-wave staging buffer (elements)
   constexpr int SW = kWave * R + (GSTAGE ? Vec16<T>::n : 0);
   const int tid = threadIdx.x;
-  const int cps = 1 << cps_log2;
+  const int cps_log2 = chunks;  // (ORDER 0)
+  const int cps = ORDER == 0 ? 1 << chunks : chunks;
   const int spb = 1 << spb_log2;
   int k, slot;
   if (ORDER == 0) {

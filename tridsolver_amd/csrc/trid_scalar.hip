@@ -144,6 +144,8 @@ PartCfg default_cfg(int order, const SysDesc &D, int vec, bool gvec, bool dense)
   if (order == 1 && cfg.kind == 1) {
     const PartCfg s = strided_default(D.N, sizeof(T));
     if (s.kind == 1) cfg = s;
+    const PartCfg w = strided_wide(D.N, D.nsys, sizeof(T));
+    if (w.kind == 1) cfg = w;
   }
   // staging pays when a chunk is more than one 16-byte vector
   if (cfg.R * sizeof(T) > 16) {
