@@ -548,6 +548,15 @@ tridStatus_t solve(const T *a, const int *a_pads, const T *b,
   // cache policy: the tuned one, else the footprint rule; a forced policy
   // wins; fallback and 64-bit-offset solves always stream
   if (!tuned) cfg.cp = cp_rule;
+  // one launch along solvedim 0 over arrays past the cache's own 256 MiB: the
+  // coefficients stream, so that they do not push d out of it.  Cached /
+  // mixed, the same arrays again and others in turn: [256, 256, 160] FP64,
+  // 320 MiB: 65 / 64 and 81 / 64 us, [300, 390, 170] FP32, 303 MiB: 63 / 62
+  // and 79 / 62, [200, 180, 250] FP64 Inc, 343 MiB: 74 / 68 and 84 / 79.
+  // Strided rows keep cached up to the rule's 384 MiB: [180, 200, 250] FP64,
+  // 275 MiB, solvedim 1: 64 / 78 and 78 / 78
+  if (!tuned && order == 0 && cfg.kind == 1 && cfg.cp == kCached && footprint > kMallBytes)
+    cfg.cp = kMixed;
   if (forced_cache_policy() >= 0) cfg.cp = forced_cache_policy();
   if (!idx32 || cfg.kind == 2) cfg.cp = kStream;
   // split-line: no mixed form, and ORDER 0 streams (2 x 2^22 rows FP64 122
