@@ -241,9 +241,9 @@ __global__ void __launch_bounds__(256)
 //   sweep term    G1_f = -lam (X_hi - X_lo) (Lam~_hi - Lam~_lo)
 //   stencil term  G_f  =  lam (Lx~_lo - Lx~_hi),  G2_f = G_f (u_hi - u_lo)
 // and gk_lo, gk_hi += (G1_f + G2_f) / 2,  ubar_hi += G_f kf,  ubar_lo -= G_f kf.
-// Launched on a (64, 4) thread tile per (x-tile, 4 rows, ZC planes): rows
-// y-1 and y+1 of the tile's interior rows come from the same work-group's
-// lines.  Each thread marches along z over ZC planes of one (x, y) column: U, K,
+// Launched on a (64, 4) or (32, 8) thread tile per (x-tile, rows, ZC planes):
+// rows y-1 and y+1 of the tile's interior rows come from the same
+// work-group's lines.  Each thread marches along z over ZC planes of one (x, y) column: U, K,
 // LX, U1 and LZ of planes z-1, z, z+1 roll through registers, so each point
 // loads the z-neighbour values once (28 loads per point instead of 38 for a
 // thread per point) and the neighbour planes never come back from L2 or HBM.
@@ -266,8 +266,8 @@ __global__ void __launch_bounds__(256)
   const unsigned t = b < nb8 ? (b & 7u) * (nb8 >> 3) + (b >> 3) : b;
   const int tx = (int)(t % (unsigned)ntx), tyz = (int)(t / (unsigned)ntx);
   const int ty = tyz % nty, tz = tyz / nty;
-  const int x = tx * 64 + threadIdx.x;
-  const int y = ty * 4 + threadIdx.y;
+  const int x = tx * (int)blockDim.x + threadIdx.x;
+  const int y = ty * (int)blockDim.y + threadIdx.y;
   if (x >= g.nx || y >= g.ny) return;
   const int z0 = tz * ZC;
   const int z1 = z0 + ZC < g.nz ? z0 + ZC : g.nz;
@@ -400,10 +400,6 @@ namespace {
 
 unsigned blocks_for(long long n) { return (unsigned)((n + 255) / 256); }
 
-// planes per thread of the gradient gather (k_vadi_grad_col; at 128^3, 16
-// planes: 54.5 -> 48 us per step, against 8 planes 50 us)
-constexpr int kGradZ = 16;
-
 Grid make_grid(int nx, int ny, int nz) {
   Grid g;
   g.nx = nx;
@@ -412,6 +408,31 @@ Grid make_grid(int nx, int ny, int nz) {
   g.nxy = (long long)nx * ny;
   g.n = g.nxy * nz;
   return g;
+}
+
+// Launch of the gradient gather: bx x (256 / bx) threads, zc planes each.
+struct GradLaunch {
+  int bx, zc, tx, ty;
+  unsigned blocks;
+};
+
+// Tile rows of 32 points where those cover the line more tightly than rows of
+// 64, and the most planes per thread that leave 1024 work-groups: fewer
+// planes re-read more of their neighbours, fewer work-groups leave the march
+// along z a serial chain on an idle chip.  Loss and gradient of 8 steps with
+// 64 x 4 x 16 tiles -> these: 26^3 587 -> 469 us, 64^3 585 -> 509, 96^3 1044
+// -> 943, 113^3 1366 -> 1348; 128^3 (8 planes) unchanged.
+GradLaunch grad_launch(const Grid &g) {
+  GradLaunch l;
+  l.bx = (g.nx + 31) / 32 * 32 < (g.nx + 63) / 64 * 64 ? 32 : 64;
+  const int by = 256 / l.bx;
+  l.tx = (g.nx + l.bx - 1) / l.bx;
+  l.ty = (g.ny + by - 1) / by;
+  const long long tiles = (long long)l.tx * l.ty;
+  l.zc = 16;
+  while (l.zc > 1 && tiles * ((g.nz + l.zc - 1) / l.zc) < 1024) l.zc >>= 1;
+  l.blocks = (unsigned)(tiles * ((g.nz + l.zc - 1) / l.zc));
+  return l;
 }
 
 SysDesc line_desc(const Grid &g, int axis) {
@@ -453,6 +474,17 @@ tridStatus_t vadi_sweep(const double *K, double *d, double *u, double *out, cons
   const int order = axis == 0 ? 0 : 1;
   PartCfg cfg = heuristic(order, D.N, 0, sizeof(double));
   if (cfg.kind != 1) return fail(TRID_STATUS_INVALID_VALUE, "vadi: grid too long along an axis");
+  // grids of up to 2^21 points leave the chip part idle: shorter chunks and
+  // smaller work-groups put more of them on it.  Loss and gradient of 8
+  // steps, heuristic -> this: y and z sweeps of 40^3 616 -> 553 us (4-row
+  // chunks, 8 systems), 64^3 585 -> 507, 96^3 1044 -> 999 (8 rows, 16
+  // systems), 128^3 1203 -> 1182; x sweeps (4 rows) 96^3 1044 -> 995, 113^3
+  // 1366 -> 1268
+  if (g.n <= 1LL << 21) {
+    PartCfg t = make_cfg(order, order == 0 || D.N <= 64 ? 4 : 8, D.N, 0, 256);
+    if (order == 1) t.spb_log2 = D.N <= 64 ? 3 : 4;
+    if (cfg_valid(t, D.N)) cfg = t;
+  }
   cfg.vec = 0;
   cfg.idx32 = (unsigned long long)g.n * 8 < (1ULL << 32) && !wide_index();
   cfg.cp = cfg.idx32 ? vadi_policy(g) : kStream;
@@ -651,9 +683,7 @@ EXTERN_C tridStatus_t tridVadiLossGrad(const double *kappa, const double *u0,
   s = check_hip(hipGetLastError(), "loss launch");
   if (s) return s;
 
-  const int grad_tx = (nx + 63) / 64, grad_ty = (ny + 3) / 4;
-  const unsigned grad_grid =
-      (unsigned)grad_tx * (unsigned)grad_ty * (unsigned)((nz + kGradZ - 1) / kGradZ);
+  const GradLaunch gl = grad_launch(g);
   for (int sg = nseg - 1; sg >= 0 && !s; sg--) {
     const int k0 = sg * ckpt, k1 = std::min(steps, k0 + ckpt);
     if (sg < nseg - 1) s = record(sg);
@@ -663,8 +693,20 @@ EXTERN_C tridStatus_t tridVadiLossGrad(const double *kappa, const double *u0,
       if (!s) s = vadi_sweep(kappa, LZ, nullptr, LY, g, 1, lam, 1, 0, st);
       if (!s) s = vadi_xT(kappa, LY, LX, g, lam, st);
       if (s) break;
-      hipLaunchKernelGGL(k_vadi_grad_col<kGradZ>, dim3(grad_grid), dim3(64, 4), 0, st, kappa, us[i],
-                         us[i + 1], P[i], Q[i], LZ, LY, LX, ubar, grad_kappa, g, lam, grad_tx, grad_ty);
+#define TRID_GRAD(ZZ)                                                                           \
+  case ZZ:                                                                                      \
+    hipLaunchKernelGGL(k_vadi_grad_col<ZZ>, dim3(gl.blocks), dim3(gl.bx, 256 / gl.bx), 0, st,   \
+                       kappa, us[i], us[i + 1], P[i], Q[i], LZ, LY, LX, ubar, grad_kappa, g,    \
+                       lam, gl.tx, gl.ty);                                                      \
+    break;
+      switch (gl.zc) {
+        TRID_GRAD(1)
+        TRID_GRAD(2)
+        TRID_GRAD(4)
+        TRID_GRAD(8)
+        TRID_GRAD(16)
+      }
+#undef TRID_GRAD
       s = check_hip(hipGetLastError(), "vadi gradient launch");
     }
   }
