@@ -755,6 +755,33 @@ struct CoefConst {
 //                   interior to the grid, a_i = -lam kf_{i-1/2},
 //                   c_i = -lam kf_{i+1/2}, b_i = 1 - a_i - c_i (identity rows
 //                   elsewhere); with transpose, its transposed operator.
+// Rows row0 .. row0+R-1 of that operator from k = kappa of rows row0-1 ..
+// row0+R (0 off the line).
+template <typename T, int R>
+__device__ __forceinline__ void kappa_rows(const T (&k)[R + 2], int row0, int N, bool line_in,
+                                           T lam, bool transpose, T (&a)[R], T (&b)[R],
+                                           T (&c)[R]) {
+  auto inner = [&](int row) { return line_in && row >= 1 && row + 2 <= N; };
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int row = row0 + r;
+    const T am = -lam * (T(0.5) * (k[r + 1] + k[r]));      // -lam kf_{row-1/2}
+    const T cp = -lam * (T(0.5) * (k[r + 1] + k[r + 2]));  // -lam kf_{row+1/2}
+    const bool in = inner(row);
+    b[r] = in ? T(1) - am - cp : T(1);
+    if (!transpose) {
+      a[r] = in ? am : T(0);
+      c[r] = in ? cp : T(0);
+    } else {
+      // (A^T)_{row,row-1} = c_{row-1} = -lam kf_{row-1/2} if row-1 is an
+      // interior row; (A^T)_{row,row+1} = a_{row+1} = -lam kf_{row+1/2}
+      a[r] = inner(row - 1) ? am : T(0);
+      c[r] = inner(row + 1) ? cp : T(0);
+      if (row >= N) b[r] = T(1);
+    }
+  }
+}
+
 template <typename T>
 struct CoefKappa {
   static constexpr bool kArrays = false;
@@ -772,25 +799,7 @@ struct CoefKappa {
       const int row = row0 - 1 + r;
       k[r] = (row >= 0 && row < N) ? *at(K, off + (I)row * s) : T(0);
     }
-    auto inner = [&](int row) { return line_in && row >= 1 && row + 2 <= N; };
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int row = row0 + r;
-      const T am = -lam * (T(0.5) * (k[r + 1] + k[r]));      // -lam kf_{row-1/2}
-      const T cp = -lam * (T(0.5) * (k[r + 1] + k[r + 2]));  // -lam kf_{row+1/2}
-      const bool in = inner(row);
-      b[r] = in ? T(1) - am - cp : T(1);
-      if (!transpose) {
-        a[r] = in ? am : T(0);
-        c[r] = in ? cp : T(0);
-      } else {
-        // (A^T)_{row,row-1} = c_{row-1} = -lam kf_{row-1/2} if row-1 is an
-        // interior row; (A^T)_{row,row+1} = a_{row+1} = -lam kf_{row+1/2}
-        a[r] = inner(row - 1) ? am : T(0);
-        c[r] = inner(row + 1) ? cp : T(0);
-        if (row >= N) b[r] = T(1);
-      }
-    }
+    kappa_rows<T, R>(k, row0, N, line_in, lam, transpose != 0, a, b, c);
   }
 };
 

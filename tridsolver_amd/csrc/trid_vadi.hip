@@ -16,6 +16,7 @@
 //     the wave's LDS buffer in 16-byte pieces; MODE 0 builds r = D u in
 //     registers and solves A_x (the right-hand side never goes to memory),
 //     MODE 1 solves the transposed system A_x^T.
+//   k_vadi_xl<R, MODE>: the same for lines of any length up to 576 points.
 //   y and z sweeps: the partitioned Thomas kernel with the CoefKappa loader
 //     (coefficients formed in registers from kappa), forward or transposed;
 //     the z sweep adds into u, optionally out of place (u_{k+1} into a new
@@ -66,6 +67,21 @@ __device__ __forceinline__ void grid_coords(const Grid &g, long long p, int &i, 
   }
 }
 
+// The stencil's right-hand side at point p, neighbours at strides st.
+__device__ __forceinline__ double vadi_stencil(const double *__restrict__ K,
+                                               const double *__restrict__ u, long long p,
+                                               const long long (&st)[3], double lam) {
+  double s = 0.0;
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const long long q = st[a];
+    const double kp = 0.5 * (K[p] + K[p + q]);
+    const double km = 0.5 * (K[p] + K[p - q]);
+    s += kp * (u[p + q] - u[p]) - km * (u[p] - u[p - q]);
+  }
+  return lam * s;
+}
+
 // r = lam * sum_axes [kf+ (u+ - u) - kf- (u - u-)] at interior points, 0 else
 __global__ void __launch_bounds__(256)
     k_vadi_rhs(const double *__restrict__ K, const double *__restrict__ u,
@@ -79,15 +95,7 @@ __global__ void __launch_bounds__(256)
     return;
   }
   const long long st[3] = {1, g.nx, g.nxy};
-  double s = 0.0;
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    const long long q = st[a];
-    const double kp = 0.5 * (K[p] + K[p + q]);
-    const double km = 0.5 * (K[p] + K[p - q]);
-    s += kp * (u[p + q] - u[p]) - km * (u[p] - u[p - q]);
-  }
-  r[p] = lam * s;
+  r[p] = vadi_stencil(K, u, p, st, lam);
 }
 
 // x sweep over whole lines, one wave holding 64/cps lines of one z-plane
@@ -232,6 +240,104 @@ __global__ void __launch_bounds__(256)
   double y[R];
   chunk_expand<double, R>(a, c, d, xf, xl, y);
   if (wave_active) store_chunk_staged<double, R, CP>(out + wo, stage, lane, y, false);
+}
+
+// x sweep over whole lines of any length up to 64 R, arrays of any alignment:
+// a wave takes 64 / cps lines of cps chunks, one contiguous span of the grid.
+// Modes as k_vadi_x.  The span's elements are read (MODE 0: the stencil is
+// evaluated) in consecutive lanes and pass through the wave's LDS buffers
+// into chunks, with kappa beside them; R is odd, which keeps the per-lane
+// chunk accesses off each other's banks.
+// Latency and launches bound it at ordinary sizes (96^3: 21 MB of kappa, u
+// and p); it replaces the right-hand-side kernel and a sweep that read its
+// rows per lane, 8.4 + 10 us at 96^3 FP64, by one launch of 13 us (MODE 1:
+// 10 -> 9.5 us).
+// One or four waves per work-group; waves past the last line leave at once.
+template <int R, int MODE>
+__global__ void __launch_bounds__(256)
+    k_vadi_xl(const double *__restrict__ K, const double *__restrict__ in,
+              double *__restrict__ out, Grid g, double lam, int cps_log2, int stream) {
+  constexpr int SW = kWave * R;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x >> 6;
+  double *sd = reinterpret_cast<double *>(smem_raw) + wv * 2 * SW, *sk = sd + SW;
+  const int cps = 1 << cps_log2, per = kWave >> cps_log2;
+  const long long nlines = (long long)g.ny * g.nz;
+  const long long line0 = ((long long)blockIdx.x * (blockDim.x >> 6) + wv) * per;
+  if (line0 >= nlines) return;  // (no work-group barrier below)
+  const int nact = nlines - line0 < per ? (int)(nlines - line0) : per;
+  const int len = nact * g.nx;  // <= 64 R
+  const long long p0 = line0 * g.nx;
+  const int k0 = (int)(line0 / g.ny), j0 = (int)(line0 - (long long)k0 * g.ny);
+  // grid line of the wave's line l
+  auto line_jk = [&](int l, int &j, int &k) {
+    j = j0 + l;
+    k = k0;
+    while (j >= g.ny) {
+      j -= g.ny;
+      k++;
+    }
+  };
+  // loads without branches, so that those of several elements are in flight
+  // together: lanes past the span read its first element, points off the
+  // interior read themselves (96^3, under branches: 15.5 us)
+#pragma unroll
+  for (int v = 0; v < R; v++) {
+    const int e = v * kWave + lane;
+    const long long p = p0 + (e < len ? e : 0);
+    const double kp = K[p];
+    double x;
+    if constexpr (MODE == 0) {
+      const int l = (int)((unsigned)(e < len ? e : 0) / (unsigned)g.nx);
+      int j, k;
+      line_jk(l, j, k);
+      const bool inp = grid_interior(g, (e < len ? e : 0) - l * g.nx, j, k);
+      const long long st[3] = {inp ? 1 : 0, inp ? g.nx : 0, inp ? g.nxy : 0};
+      x = vadi_stencil(K, in, p, st, lam);
+      if (!inp) x = 0.0;  // (also where the point's own values are not finite)
+    } else {
+      x = in[p];
+    }
+    if (e < len) {
+      sd[e] = x;
+      sk[e] = kp;
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+  const int c = lane & (cps - 1), slot = lane >> cps_log2;
+  const bool on = slot < nact;
+  int j, k;
+  line_jk(on ? slot : 0, j, k);
+  const bool line_in = on && j >= 1 && j <= g.ny - 2 && k >= 1 && k <= g.nz - 2;
+  const int row0 = c * R, N = on ? g.nx : 0, i0 = slot * g.nx + row0;
+  double kc[R + 2], a[R], b[R], cc[R], d[R];
+#pragma unroll
+  for (int r = 0; r < R + 2; r++) {
+    const int row = row0 - 1 + r;
+    kc[r] = row >= 0 && row < N ? sk[i0 - 1 + r] : 0.0;
+  }
+#pragma unroll
+  for (int r = 0; r < R; r++) d[r] = row0 + r < N ? sd[i0 + r] : 0.0;
+  kappa_rows<double, R>(kc, row0, N, line_in, lam, MODE == 1, a, b, cc);
+  Row<double> f, l;
+  chunk_reduce<double, R>(a, b, cc, d, f, l);
+  double xf, xl;
+  reduced_wave<double>(f, l, c, cps, lane, xf, xl);
+  double y[R];
+  chunk_expand<double, R>(a, cc, d, xf, xl, y);
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if (row0 + r < N) sd[i0 + r] = y[r];
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int v = 0; v < R; v++) {
+    const int e = v * kWave + lane;
+    if (e < len) {
+      if (stream) st_stream<kStream>(out + p0 + e, sd[e]);
+      else out[p0 + e] = sd[e];
+    }
+  }
 }
 
 // Adjoint of one step at every point p (gather form, no atomics).  For each
@@ -539,11 +645,54 @@ tridStatus_t launch_vadi_x(int R, const double *K, const double *in, double *out
   return check_hip(hipGetLastError(), "vadi x launch");
 }
 
+// Chunk length of k_vadi_xl for lines of nx points (0: too long).  Chunks are
+// a power of two per line; short ones keep the wave's element-wise phase and
+// its chains short, which counts most on small grids (loss and gradient of 8
+// steps, 3 / 5 / 7 / 9 rows: 33^3 414 / 425 / 438 / 462 us, 80^3 679 / 659 /
+// 668 / 684, 96^3 782 / 799 / 807 / 818, 113^3 1306 / 1275 / 1307 / 1313):
+// 3 rows up to 64 points, then whichever of 3 and 5 (past 160 points 5, 7
+// and 9) pads the line least.
+int line_x_rows(int nx) {
+  if (nx <= 64) return 3;
+  int best = 0;
+  for (int R : {3, 5, 7, 9}) {
+    const int cps = 1 << ilog2((nx + R - 1) / R);
+    if (cps > (R == 3 ? 32 : kWave) || (nx <= 160 && R > 5)) continue;
+    if (!best || cps * R < best * (1 << ilog2((nx + best - 1) / best))) best = R;
+  }
+  return best;
+}
+
+template <int MODE>
+tridStatus_t launch_vadi_xl(int R, const double *K, const double *in, double *out, const Grid &g,
+                            double lam, hipStream_t st) {
+  const int cl = ilog2((g.nx + R - 1) / R), per = kWave >> cl;
+  const long long waves = ((long long)g.ny * g.nz + per - 1) / per;
+  // single-wave work-groups spread a small grid over more CUs
+  const int wpb = waves >= 2048 ? 4 : 1;
+  const dim3 blocks((unsigned)((waves + wpb - 1) / wpb)), threads(wpb * kWave);
+  const int stream = vadi_policy(g) == kStream;
+#define TRID_XL(RR)                                                                          \
+  case RR:                                                                                   \
+    hipLaunchKernelGGL((k_vadi_xl<RR, MODE>), blocks, threads, wpb * 2 * kWave * RR * 8, st, K, \
+                       in, out, g, lam, cl, stream);                                         \
+    break;
+  switch (R) {
+    TRID_XL(3)
+    TRID_XL(5)
+    TRID_XL(7)
+    TRID_XL(9)
+  }
+#undef TRID_XL
+  return check_hip(hipGetLastError(), "vadi x line launch");
+}
+
 // p = A_x^{-1} D(kappa) u   (r: scratch for the unfused path; may equal p)
 tridStatus_t vadi_rhs_x(const double *K, const double *u, double *p, const Grid &g, double lam,
                         hipStream_t st) {
   const int R = staged_x_rows(g, K, u, p);
   if (R) return launch_vadi_x<0>(R, K, u, p, g, lam, st);
+  if (const int rl = line_x_rows(g.nx)) return launch_vadi_xl<0>(rl, K, u, p, g, lam, st);
   tridStatus_t s = vadi_rhs(K, u, p, g, lam, st);
   if (!s) s = vadi_sweep(K, p, nullptr, nullptr, g, 0, lam, 0, 0, st);
   return s;
@@ -554,6 +703,7 @@ tridStatus_t vadi_xT(const double *K, double *in, double *out, const Grid &g, do
                      hipStream_t st) {
   const int R = staged_x_rows(g, K, in, out);
   if (R) return launch_vadi_x<1>(R, K, in, out, g, lam, st);
+  if (const int rl = line_x_rows(g.nx)) return launch_vadi_xl<1>(rl, K, in, out, g, lam, st);
   return vadi_sweep(K, in, nullptr, out, g, 0, lam, 1, 0, st);
 }
 
