@@ -18,12 +18,21 @@ from . import _check, lib
 from .api import _iv, dims_of, solve
 
 
+def _sync(t) -> int:
+    """0 where the library launches on the stream that torch works on for t's
+    device: what follows there is ordered behind the call, and so is the reuse
+    of its temporaries; elsewhere 1, and the call waits for its results.
+    The waits kept the host from preparing the next launch: forward and
+    backward of 1000 x 4000 FP32 took 176 us for 58 us of kernels."""
+    return int((lib().tridGetStream() or 0) != torch.cuda.current_stream(t.device).cuda_stream)
+
+
 class TridSolve(torch.autograd.Function):
     @staticmethod
     def forward(ctx, a, b, c, d, solvedim: int):
         x = d.detach().clone().contiguous()
         solve(a.detach().contiguous(), b.detach().contiguous(), c.detach().contiguous(), x,
-              solvedim)
+              solvedim, sync=_sync(x))
         ctx.solvedim = solvedim
         ctx.save_for_backward(a, b, c, x)
         return x
@@ -38,7 +47,7 @@ class TridSolve(torch.autograd.Function):
               else lib().tridSmtsvStridedBatchAdjoint)
         _check(fn(a.data_ptr(), b.data_ptr(), c.data_ptr(), x.data_ptr(), gx.data_ptr(),
                   ga.data_ptr(), gb.data_ptr(), gc.data_ptr(), gd.data_ptr(), len(dims),
-                  ctx.solvedim, _iv(dims), _iv(dims), 1), "tridXmtsvStridedBatchAdjoint")
+                  ctx.solvedim, _iv(dims), _iv(dims), _sync(x)), "tridXmtsvStridedBatchAdjoint")
         return ga, gb, gc, gd, None
 
 
