@@ -877,6 +877,15 @@ __host__ __device__ constexpr bool blk2tw_sizes(int M) { return M >= 3 && M <= 8
 // layout code of the two-ended tiled kernel (tridBlkForceLanes, MixedArgs::L)
 constexpr int kTwistTiled = 200;
 
+// Rows that a wave of the two-ended tiled kernel has on their way while it
+// eliminates one.  A half's rows are a serial chain, each step at least a
+// load's latency: with two rows on their way M = 4 and 5 FP64, N = 100, P =
+// 600 take 81 and 110 us against 93 and 115 (four-wave work-groups; one-wave
+// ones 59 and 82).  M = 3 has small blocks, of which waves re-read shared
+// cache lines (P = 8000: 133 against 112 us), and M >= 6 no registers for a
+// second row.
+__host__ __device__ constexpr int blk2_tw_ahead(int M) { return M == 4 || M == 5 ? 2 : 1; }
+
 // Two-ended form of blk2_problem (the elimination of blk_problem_tw with the
 // tiled kernel's cooperative block moves): two groups of M lanes per
 // problem, each with its own tile.  Half 0 eliminates rows 0 .. m-1
@@ -914,40 +923,43 @@ __device__ __forceinline__ void blk2_problem_tw(const BlkArgs<T> &g, long long p
     Cp[i] = T(0);
     dp[i] = T(0);
   }
-  // this lane's elements j, j+M, ... of the next row's K, B, F blocks and
-  // entry j of its d (the next row is loaded while this one is eliminated)
-  T rk[M], rb[M], rf[M], rd;
-  auto load_step = [&](int s) {
-    const int n = rowof(s);
-#pragma unroll
-    for (int r = 0; r < M; r++) {
-      const int e = j + M * r;
-      rk[r] = s > 0 ? (h == 0 ? ld_sub(n, e) : ld_sup(n, e)) : T(0);
-      rb[r] = g.B[blk(n) + e];
-      rf[r] = h == 0 ? ld_sup(n, e) : ld_sub(n, e);
-    }
-    rd = g.d[vec(n) + j];
+  // this lane's elements j, j+M, ... of a coming row's K, B, F blocks and
+  // entry j of its d: rows 0 .. cnt-1 of the half, then the middle row
+  struct Ahead {
+    T k[M], b[M], f[M], d;
   };
-  auto load_mid = [&]() {
+  auto load_row = [&](int s, Ahead &w) {
+    if (s < cnt) {
+      const int n = rowof(s);
 #pragma unroll
-    for (int r = 0; r < M; r++) {
-      const int e = j + M * r;
-      rk[r] = m > 0 ? ld_sub(m, e) : T(0);
-      rb[r] = g.B[blk(m) + e];
-      rf[r] = m < N - 1 ? ld_sup(m, e) : T(0);
+      for (int r = 0; r < M; r++) {
+        const int e = j + M * r;
+        w.k[r] = s > 0 ? (h == 0 ? ld_sub(n, e) : ld_sup(n, e)) : T(0);
+        w.b[r] = g.B[blk(n) + e];
+        w.f[r] = h == 0 ? ld_sup(n, e) : ld_sub(n, e);
+      }
+      w.d = g.d[vec(n) + j];
+    } else if (s == cnt) {
+#pragma unroll
+      for (int r = 0; r < M; r++) {
+        const int e = j + M * r;
+        w.k[r] = m > 0 ? ld_sub(m, e) : T(0);
+        w.b[r] = g.B[blk(m) + e];
+        w.f[r] = m < N - 1 ? ld_sup(m, e) : T(0);
+      }
+      w.d = g.d[vec(m) + j];
     }
-    rd = g.d[vec(m) + j];
   };
-  auto put_tiles = [&]() {
+  auto put_tiles = [&](const Ahead &w) {
     if (lane_ok) {
 #pragma unroll
       for (int r = 0; r < M; r++) {
         const int e = j + M * r;
-        sK[e] = rk[r];
-        sB[e] = rb[r];
-        sF[e] = rf[r];
+        sK[e] = w.k[r];
+        sB[e] = w.b[r];
+        sF[e] = w.f[r];
       }
-      sd[j] = rd;
+      sd[j] = w.d;
     }
     wb();
   };
@@ -989,13 +1001,16 @@ __device__ __forceinline__ void blk2_problem_tw(const BlkArgs<T> &g, long long p
     }
   };
 
-  if (cnt > 0) load_step(0);
-  else load_mid();
-  for (int s = 0; s < cnt; s++) {
+  // D rows are on their way while one is eliminated; row s is in w[s % D]
+  // (constant indices: a register that waits for its load cannot be moved)
+  constexpr int D = blk2_tw_ahead(M);
+  Ahead w[D];
+#pragma unroll
+  for (int t = 0; t < D; t++) load_row(t, w[t]);
+  auto step = [&](int s, Ahead &wr) {
     const int n = rowof(s);
-    put_tiles();
-    if (s + 1 < cnt) load_step(s + 1);
-    else load_mid();
+    put_tiles(wr);
+    load_row(s + D, wr);
     T X[M], Cn[M], v[M];
 #pragma unroll
     for (int i = 0; i < M; i++) {
@@ -1025,6 +1040,11 @@ __device__ __forceinline__ void blk2_problem_tw(const BlkArgs<T> &g, long long p
       Cp[i] = Cn[i];
       dp[i] = v[i];
     }
+  };
+  for (int s = 0; s < cnt; s += D) {
+#pragma unroll
+    for (int t = 0; t < D; t++)
+      if (s + t < cnt) step(s + t, w[t]);
   }
 
   // the middle row: the upper neighbour's C', d' and the lower one's A'',
@@ -1035,7 +1055,11 @@ __device__ __forceinline__ void blk2_problem_tw(const BlkArgs<T> &g, long long p
     Qo[i] = lane_read(Cp[i], partner);
     qo[i] = lane_read(dp[i], partner);
   }
-  put_tiles();
+  if constexpr (D == 2) {
+    // (the halves' counts differ by one when N is even)
+    if (cnt & 1) w[0] = w[1];
+  }
+  put_tiles(w[0]);
   T un[M];
   {
     T X[M], Cn[M], v[M];
@@ -1063,22 +1087,28 @@ __device__ __forceinline__ void blk2_problem_tw(const BlkArgs<T> &g, long long p
 
   // substitution outward from the middle over the half's rows: lane i forms
   // u_n[i] = d*_n[i] - F*_n[i, :] u_prev from the row's tile
-  T bc[M], bd = T(0);
-  auto load_back = [&](int n) {
-#pragma unroll
-    for (int r = 0; r < M; r++) bc[r] = g.Cs[blk(n) + j + M * r];
-    bd = g.ds[vec(n) + j];
+  struct Back {
+    T c[M], d;
   };
-  if (cnt > 0) load_back(rowof(cnt - 1));
-  for (int s = cnt - 1; s >= 0; s--) {
+  auto load_back = [&](int s, Back &v) {
+    if (s < 0) return;
     const int n = rowof(s);
-    const T dj = bd;
+#pragma unroll
+    for (int r = 0; r < M; r++) v.c[r] = g.Cs[blk(n) + j + M * r];
+    v.d = g.ds[vec(n) + j];
+  };
+  Back v[D];
+#pragma unroll
+  for (int t = 0; t < D; t++) load_back(cnt - 1 - t, v[t]);
+  auto back = [&](int s, Back &vr) {
+    const int n = rowof(s);
+    const T dj = vr.d;
     if (lane_ok) {
 #pragma unroll
-      for (int r = 0; r < M; r++) sF[j + M * r] = bc[r];
+      for (int r = 0; r < M; r++) sF[j + M * r] = vr.c[r];
     }
     wb();
-    if (s >= 1) load_back(rowof(s - 1));
+    load_back(s - D, vr);
     T acc = dj;
 #pragma unroll
     for (int k = 0; k < M; k++) acc -= sF[j * M + k] * un[k];
@@ -1088,6 +1118,11 @@ __device__ __forceinline__ void blk2_problem_tw(const BlkArgs<T> &g, long long p
     for (int k = 0; k < M; k++) un[k] = su[k];
     wb();
     if (store) g.u[vec(n) + j] = acc;
+  };
+  for (int s = cnt - 1; s >= 0; s -= D) {
+#pragma unroll
+    for (int t = 0; t < D; t++)
+      if (s - t >= 0) back(s - t, v[t]);
   }
 }
 
@@ -1108,7 +1143,7 @@ __device__ __forceinline__ void blk2_tw_block(const BlkArgs<T> &g, long long blo
   const int in = lane - grp * 2 * M;
   const int h = in / M, j = in - h * M;
   const bool lane_ok = grp < G2;
-  const long long p = (block * 4 + wave) * G2 + grp;
+  const long long p = (block * (long long)(blockDim.x >> 6) + wave) * G2 + grp;
   const bool store = lane_ok && p < g.P;
   // idle lanes past the last whole group read the last group's first tile,
   // solve problem P-1 again and write nothing
@@ -1122,7 +1157,11 @@ __device__ __forceinline__ void blk2_tw_block(const BlkArgs<T> &g, long long blo
 template <typename T, int M, int TRANS>
 __global__ void __launch_bounds__(256, blk2_min_waves(M)) k_blk2_tw(BlkArgs<T> g) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  blk2_tw_block<T, M, TRANS>(g, blockIdx.x, reinterpret_cast<T *>(smem_raw));
+  // XCD-contiguous order (as k_part): a wave's run of blocks ends inside a
+  // cache line that the next one's begins in
+  const unsigned nb8 = gridDim.x & ~7u, b = blockIdx.x;
+  const unsigned block = b < nb8 ? (b & 7u) * (nb8 >> 3) + (b >> 3) : b;
+  blk2_tw_block<T, M, TRANS>(g, block, reinterpret_cast<T *>(smem_raw));
 }
 
 template <typename T, int M>
@@ -1194,24 +1233,59 @@ __global__ void __launch_bounds__(256) k_blk_mixed(MixedArgs a) {
 
 // ---- adjoint gradients: outer products ------------------------------------
 // grad_A_n = -lam_n u_{n-1}^T, grad_B_n = -lam_n u_n^T, grad_C_n = -lam_n u_{n+1}^T
-// one thread per block entry (n, p, i, c)
-template <typename T>
+// One thread per entry (p, i, c) of kGradRows rows n: u_{n-1}, u_n, u_{n+1}
+// roll through registers, so a row loads one value of u and one of lam per
+// entry.  Bound by the three gradients' writes, which nothing reads again
+// soon (non-temporal).  M = 3, N = 100, P = 8000 FP64 (211 MB): 53 us with a
+// thread per entry of one row and divisions by runtime sizes, 42 us now.
+constexpr int kGradRows = 4;
+
+template <typename T, int M, typename I>
 __global__ void __launch_bounds__(256)
-    k_blk_grads(const T *__restrict__ lam, const T *__restrict__ u,
-                T *__restrict__ gA, T *__restrict__ gB, T *__restrict__ gC,
-                int N, long long P, int M) {
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long MM = (long long)M * M;
-  const long long total = (long long)N * P * MM;
-  if (e >= total) return;
-  const long long bp = e / MM;  // n * P + p
-  const int ic = (int)(e - bp * MM);
-  const int i = ic / M, c = ic - (ic / M) * M;
-  const long long n = bp / P;
-  const T l = lam[bp * M + i];
-  gB[e] = -l * u[bp * M + c];
-  gA[e] = n > 0 ? -l * u[(bp - P) * M + c] : T(0);
-  gC[e] = n < N - 1 ? -l * u[(bp + P) * M + c] : T(0);
+    k_blk_grads(const T *__restrict__ lam, const T *__restrict__ u, T *__restrict__ gA,
+                T *__restrict__ gB, T *__restrict__ gC, int N, I P) {
+  const I e = (I)blockIdx.x * 256 + threadIdx.x;
+  if (e >= P * (M * M)) return;
+  const I p = e / (M * M);
+  const int ic = (int)(e - p * (M * M)), i = ic / M, c = ic - i * M;
+  const long long rv = (long long)P * M, rb = rv * M;  // a row of vectors, of blocks
+  const long long ov = (long long)p * M, groups = (N + kGradRows - 1) / kGradRows;
+  for (long long q = blockIdx.y; q < groups; q += gridDim.y) {
+    const int n0 = (int)q * kGradRows;
+    T l[kGradRows], x[kGradRows + 2];
+#pragma unroll
+    for (int r = 0; r < kGradRows + 2; r++) {
+      const int n = n0 - 1 + r;
+      x[r] = n >= 0 && n < N ? u[n * rv + ov + c] : T(0);
+    }
+#pragma unroll
+    for (int r = 0; r < kGradRows; r++) l[r] = n0 + r < N ? lam[(n0 + r) * rv + ov + i] : T(0);
+#pragma unroll
+    for (int r = 0; r < kGradRows; r++) {
+      const int n = n0 + r;
+      if (n >= N) break;
+      const long long o = n * rb + (long long)e;
+      st_stream(gB + o, -l[r] * x[r + 1]);
+      st_stream(gA + o, n > 0 ? -l[r] * x[r] : T(0));
+      st_stream(gC + o, n < N - 1 ? -l[r] * x[r + 2] : T(0));
+    }
+  }
+}
+
+template <typename T, int M>
+hipError_t launch_blk_grads(const T *lam, const T *u, T *gA, T *gB, T *gC, int N, long long P,
+                            hipStream_t st) {
+  const long long entries = P * M * M;
+  const dim3 grid((unsigned)((entries + 255) / 256),
+                  (unsigned)std::min((N + kGradRows - 1) / kGradRows, 65535));
+  // 32-bit entry numbers, the last work-group's past the end included
+  if (entries < (1LL << 32) - 256 && !wide_index())
+    hipLaunchKernelGGL((k_blk_grads<T, M, uint32_t>), grid, dim3(256), 0, st, lam, u, gA, gB, gC,
+                       N, (uint32_t)P);
+  else
+    hipLaunchKernelGGL((k_blk_grads<T, M, long long>), grid, dim3(256), 0, st, lam, u, gA, gB, gC,
+                       N, P);
+  return hipGetLastError();
 }
 
 }  // namespace tridhip
@@ -1234,10 +1308,16 @@ hipError_t launch_m(const BlkArgs<T> &g, int lanes, hipStream_t st) {
   const int L = lanes > 0 ? lanes : Ld;
   if constexpr (blk2tw_sizes(M)) {
     if (lanes == kTwistTiled) {
-      const long long G = 4 * (kWave / (2 * M));
-      const size_t lds = blk2_tw_lds<T, M>();
-      hipLaunchKernelGGL((k_blk2_tw<T, M, TRANS>), dim3((unsigned)((g.P + G - 1) / G)), dim3(256),
-                         lds, st, g);
+      const long long waves = (g.P + kWave / (2 * M) - 1) / (kWave / (2 * M));
+      // one-wave work-groups spread a small batch over all CUs and end
+      // together (N = 100, FP64, one / four waves: M = 4, P = 2500 69 / 82 us,
+      // M = 7, P = 5000 258 / 330; P = 16384, M = 5 435 / 423); the short
+      // blocks of M = 3 share more cache lines between waves (P = 5000 71 /
+      // 85, 8000 107 / 105)
+      const int wpb = waves < (M == 3 ? 640 : 2048) ? 1 : 4;
+      const size_t lds = blk2_tw_lds<T, M>() / 4 * wpb;
+      hipLaunchKernelGGL((k_blk2_tw<T, M, TRANS>), dim3((unsigned)((waves + wpb - 1) / wpb)),
+                         dim3(wpb * kWave), lds, st, g);
       return hipGetLastError();
     }
   }
@@ -1518,10 +1598,25 @@ EXTERN_C tridStatus_t tridDbtsvAdjoint(const double *A, const double *B,
   s = check_hip(launch_blk<double, 1>(ga, M, choose_layout<double, 1>(ga, M, st), st),
                 "adjoint kernel launch");
   if (s) return s;
-  const long long total = (long long)N * P * M * M;
-  hipLaunchKernelGGL(k_blk_grads<double>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
-                     st, grad_d, u, grad_A, grad_B, grad_C, N, (long long)P, M);
-  s = check_hip(hipGetLastError(), "gradient kernel launch");
+  hipError_t e = hipErrorInvalidValue;
+  switch (M) {
+#define TRID_G(MM)                                                                          \
+  case MM:                                                                                  \
+    e = launch_blk_grads<double, MM>(grad_d, u, grad_A, grad_B, grad_C, N, (long long)P, st); \
+    break;
+    TRID_G(1)
+    TRID_G(2)
+    TRID_G(3)
+    TRID_G(4)
+    TRID_G(5)
+    TRID_G(6)
+    TRID_G(7)
+    TRID_G(8)
+    TRID_G(9)
+    TRID_G(10)
+#undef TRID_G
+  }
+  s = check_hip(e, "gradient kernel launch");
   if (s) return s;
   if (sync) return check_hip(hipStreamSynchronize(st), "hipStreamSynchronize");
   return TRID_STATUS_SUCCESS;
