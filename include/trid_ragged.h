@@ -31,16 +31,15 @@
  * the whole solve faster by more than 2 %.
  * The plan builds a work list per family ordered from the most to the least
  * expensive item; each solve is one launch of a persistent kernel per
- * family present, whose work-groups pull items from an atomic counter
- * (reset by the kernel itself).  Systems longer than 8192 rows are solved
- * after it: the longest of them one by one, each as a strided batch of one
+ * family present, whose work-groups take every grid-th item.  Systems
+ * longer than 8192 rows are solved after it: the longest of them one by one, each as a strided batch of one
  * system (tridXmtsvStridedBatch, split-line solve past 8192 rows), the rest
  * by a one-thread-per-system launch; the plan picks the split by a cost
  * model (untuned: a one-system solve ~25 us, the one-thread launch ~0.5 us
  * per row of its longest system; the autotuner measures both on the plan's
  * longest system).
- * A plan may be used for any arrays with the same offsets; calls that
- * overlap on one plan race on its counter and must be stream-ordered.
+ * A plan may be used for any arrays with the same offsets; a solve changes
+ * nothing in it.
  */
 #ifndef TRIDSOLVER_AMD_TRID_RAGGED_H
 #define TRIDSOLVER_AMD_TRID_RAGGED_H

@@ -74,7 +74,6 @@ struct RagArgs {
   const int *sys;  // system ids, grouped by bin
   const RagItem *items;
   int nitems;
-  unsigned *counter;  // [0] next item, [1] finished work-groups
 };
 
 // Span-group staging.  A span group is the G lanes that hold one contiguous
@@ -295,33 +294,21 @@ __device__ __forceinline__ void rag_dispatch(const RagArgs<T> &g, const RagItem 
   }
 }
 
-// Persistent work-groups take items from an atomic counter; the next
-// item's index is fetched while the current item is processed.  RLO..RHI:
-// the chunk lengths of the launch's items.
+// Persistent work-groups: work-group w takes items w, w + grid, ...  The list
+// is sorted by cost and items of one bin cost the same, so the shares come out
+// even without a work queue.  (One device-wide counter for the next item and
+// the finished work-groups serialised 512 groups on one address: 50000 FP64
+// systems of 4..64, 8..512 and 8..4096 rows took 71, 110 and 333 us, now 37,
+// 70 and 304; one work-group per item 36, 74 and 291.)  RLO..RHI: the chunk
+// lengths of the launch's items.
 template <typename T, int RLO, int RHI>
 __global__ void __launch_bounds__(kRagThreads) k_ragged(RagArgs<T> g) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *smem = reinterpret_cast<T *>(smem_raw);
-  __shared__ int s_next;
-  if (threadIdx.x == 0) s_next = (int)atomicAdd(g.counter, 1u);
-  __syncthreads();
-  int i = s_next;
-  while (i < g.nitems) {
-    __syncthreads();  // every lane has read s_next
-    if (threadIdx.x == 0) s_next = (int)atomicAdd(g.counter, 1u);
+  for (int i = blockIdx.x; i < g.nitems; i += gridDim.x) {
     const RagItem it = g.items[i];
     rag_dispatch<T, RLO, RHI>(g, it, smem);
-    __syncthreads();  // s_next written; the next item reuses the staging region
-    i = s_next;
-  }
-  // the last work-group to finish resets the counters for the next launch
-  if (threadIdx.x == 0) {
-    __threadfence();
-    const unsigned done = atomicAdd(g.counter + 1, 1u);
-    if (done == gridDim.x - 1) {
-      atomicExch(g.counter, 0u);
-      atomicExch(g.counter + 1, 0u);
-    }
+    __syncthreads();  // the next item reuses the staging region
   }
 }
 
@@ -399,7 +386,6 @@ struct tridRaggedPlan_st {
   long long nsys = 0;
   long long extent = 0;  // offsets[nsys]: elements every array must hold
   const int64_t *offsets = nullptr;  // caller's device array
-  unsigned *counter = nullptr;  // both launches' (each resets it at its end)
   RagLaunch launch[2];          // family 0, family 1
   int *long_ids = nullptr;
   long long *long_ws_off = nullptr;
@@ -426,7 +412,6 @@ void free_plan(tridRaggedPlan_st *p) {
   if (!p) return;
   free_launch(p->launch[0]);
   free_launch(p->launch[1]);
-  (void)hipFree(p->counter);
   (void)hipFree(p->long_ids);
   (void)hipFree(p->long_ws_off);
   delete p;
@@ -460,15 +445,18 @@ bool red_matters(int c, int f) {
   return bin_of(Lmax, f, R) > 6;
 }
 
-RagChoice default_choice(int c, bool dbl) {
-  // measured on MI355X over 200,000 systems of 8..4096 rows: FP64 runs
-  // fastest with family 0 up to 4096 rows (family 1 past it) and PCR
-  // through LDS (1.26 ms against 1.31-1.35 ms for the other three
-  // combinations); FP32 (half the registers per row) with family 1
-  // throughout and the per-wave reduced solve (0.68 ms against 0.69-0.78)
+// past_f0: the batch has systems of more than 4096 rows
+RagChoice default_choice(int c, bool dbl, bool past_f0) {
+  // measured on MI355X, us for families 0 / 1.  FP64: family 0 up to 4096
+  // rows, family 1 past it, PCR through LDS (50000 systems of 8..4096 rows
+  // 305 / 343, of 8..512 71 / 94; 24000 of 8..6000 rows 216, 224 all in
+  // family 1).  FP32: family 0 and PCR through LDS (50000 of 8..512 rows 43 /
+  // 56, 12000 of 8..4096 rows 44 / 49), unless the batch needs family 1
+  // anyway: then all of it, in one launch, with the per-wave reduced solve
+  // (24000 of 8..6000 rows 116 in two launches, 109)
   RagChoice ch;
-  ch.fam = dbl && c < 10 ? 0 : 1;
-  ch.red = dbl ? 0 : 1;
+  ch.fam = c < 10 && (dbl || !past_f0) ? 0 : 1;
+  ch.red = dbl || !past_f0 ? 0 : 1;
   return ch;
 }
 
@@ -604,14 +592,12 @@ tridStatus_t make_launch(RagLaunch &l, int f, bool dbl, const std::vector<int> &
 struct TuneBufs {
   void *a = nullptr, *b = nullptr, *c = nullptr, *d = nullptr;
   int64_t *off = nullptr;
-  unsigned *counter = nullptr;
   ~TuneBufs() {
     (void)hipFree(a);
     (void)hipFree(b);
     (void)hipFree(c);
     (void)hipFree(d);
     (void)hipFree(off);
-    (void)hipFree(counter);
   }
 };
 
@@ -698,12 +684,10 @@ tridStatus_t tune_plan(const std::vector<int64_t> &off, const std::vector<std::v
   TuneBufs tb;
   tridStatus_t s = alloc_synthetic<T>(tb, soff.back(), st);
   if (!s) s = upload((void **)&tb.off, soff.data(), soff.size() * sizeof(int64_t));
-  unsigned zero[2] = {0, 0};
-  if (!s) s = upload((void **)&tb.counter, zero, sizeof zero);
   if (s) return s;
   const RagArgs<T> g{static_cast<const T *>(tb.a), static_cast<const T *>(tb.b),
                      static_cast<const T *>(tb.c), static_cast<T *>(tb.d), nullptr, 0,
-                     tb.off, nullptr, nullptr, 0, tb.counter};
+                     tb.off, nullptr, nullptr, 0};
   auto eval = [&](const RagChoice *ch, float &ms) -> tridStatus_t {
     RagLaunch ls[2];
     tridStatus_t r = TRID_STATUS_SUCCESS;
@@ -785,7 +769,7 @@ tridStatus_t tune_long(long long Lmax, double &solo_us, double &row_us, hipStrea
   if (!s) {
     T *a = static_cast<T *>(tb.a), *b = static_cast<T *>(tb.b), *c = static_cast<T *>(tb.c),
       *d = static_cast<T *>(tb.d);
-    RagArgs<T> g{a, b, c, d, nullptr, 0, tb.off, nullptr, nullptr, 0, nullptr};
+    RagArgs<T> g{a, b, c, d, nullptr, 0, tb.off, nullptr, nullptr, 0};
     int dims[1] = {(int)Lmax}, opts[1] = {0};
     std::vector<float> tm;
     auto prep = [&](int) { return true; };
@@ -823,9 +807,7 @@ tridStatus_t ragged_solve(tridRaggedPlan_st *p, const T *a, const T *b, const T 
   if (!a || !b || !c || !d || (inc && !u))
     return fail(TRID_STATUS_INVALID_VALUE, "NULL array");
   hipStream_t st = current_stream();
-  RagArgs<T> g{a, b, c, d, u, inc ? 1 : 0, p->offsets, nullptr, nullptr, 0, p->counter};
-  // the two launches are stream-ordered: the first one's last work-group
-  // has reset the counter when the second starts
+  RagArgs<T> g{a, b, c, d, u, inc ? 1 : 0, p->offsets, nullptr, nullptr, 0};
   for (int f = 0; f < 2; f++) {
     tridStatus_t s = check_hip(launch_family<T>(f, p->launch[f], g, st), "ragged kernel launch");
     if (s) return s;
@@ -940,7 +922,7 @@ tridStatus_t create_plan(tridRaggedPlan_st *p, const std::vector<int64_t> &off) 
   // a row family and reduced solve per length class
   RagChoice choice[kRagClasses];
   for (int c = 0; c < kRagClasses; c++) {
-    choice[c] = default_choice(c, dbl);
+    choice[c] = default_choice(c, dbl, !cls[10].empty());
     if (forced.fam >= 0 && fam_ok(c, forced.fam)) choice[c].fam = forced.fam;
     if (forced.red >= 0) choice[c].red = forced.red;
   }
@@ -980,10 +962,6 @@ tridStatus_t create_plan(tridRaggedPlan_st *p, const std::vector<int64_t> &off) 
   p->long_ws = lws;
   tridStatus_t s = upload((void **)&p->long_ids, longs.data(), longs.size() * sizeof(int));
   if (!s) s = upload((void **)&p->long_ws_off, long_off.data(), long_off.size() * sizeof(long long));
-  if (!s) {
-    unsigned zero[2] = {0, 0};
-    s = upload((void **)&p->counter, zero, sizeof zero);
-  }
   return s;
 }
 
