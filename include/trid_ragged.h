@@ -22,8 +22,8 @@
  * past 64 chunks, one of two reduced solves: PCR through LDS, one barrier per
  * level, or PCR within each wave followed by a serial sweep across the
  * waves (three barriers).  Untuned, FP64 takes 5..8 rows up to 4096 rows with
- * PCR through LDS, FP32 (half the registers per row) 9..16 rows throughout
- * with the per-wave reduced solve.  With the autotuner on (tridSetAutotune(1)
+ * PCR through LDS, FP32 the same unless a system has more than 4096 rows:
+ * then 9..16 rows throughout with the per-wave reduced solve.  With the autotuner on (tridSetAutotune(1)
  * when the plan is created) the plan times whole solves of a synthetic batch
  * with its own lengths (a uniform sample of the systems past 2^27 unknowns),
  * in buffers of its own, and from the untuned choices changes one class at a

@@ -276,12 +276,8 @@ __device__ __forceinline__ void reduced_lds_w(const Row<T> &f, const Row<T> &l, 
   sm[5 * n + me] = l.d;
   __syncthreads();
   const int lane = threadIdx.x & (kWave - 1);
-  const int per = kWave / cps;  // systems per wave and turn
-  const int s1 = lane / cps, k2 = lane - s1 * cps;
-  const int step = (int)(blockDim.x >> 6) * per;
-  for (int s0 = (int)(threadIdx.x >> 6) * per; s0 < spb; s0 += step) {
-    const bool on = s1 < per && s0 + s1 < spb;
-    const int e = on ? k2 * sp + s0 + s1 : 0;
+  auto turn = [&](int k2, int s2, bool on) {
+    const int e = on ? k2 * sp + s2 : 0;
     const Row<T> f2{sm[e], sm[n + e], sm[2 * n + e]};
     const Row<T> l2{sm[3 * n + e], sm[4 * n + e], sm[5 * n + e]};
     T xf2, xl2;
@@ -290,6 +286,17 @@ __device__ __forceinline__ void reduced_lds_w(const Row<T> &f, const Row<T> &l, 
       sm[e] = xf2;
       sm[n + e] = xl2;
     }
+  };
+  const int wave = threadIdx.x >> 6;
+  if ((cps & (cps - 1)) == 0) {
+    // every lane is in a system and one turn takes them all
+    const int cl = __builtin_ctz(cps);
+    turn(lane & (cps - 1), wave * (kWave >> cl) + (lane >> cl), true);
+  } else {
+    const int per = kWave / cps;  // systems per wave and turn
+    const int s1 = lane / cps, step = (int)(blockDim.x >> 6) * per;
+    for (int s0 = wave * per; s0 < spb; s0 += step)
+      turn(lane - s1 * cps, s0 + s1, s1 < per && s0 + s1 < spb);
   }
   __syncthreads();
   xf = sm[me];
