@@ -1,0 +1,85 @@
+"""What the differentiable wrappers hand to the library, on the CPU: the
+library is replaced by one that solves with the oracle over the addresses it
+is given."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from tests.helpers import dd_system, oracle_solve
+from tridsolver_amd import autograd
+
+
+class OracleLib:
+    """The adjoint entry points over host arrays."""
+
+    def _adjoint(self, a, b, c, x, g, ga, gb, gc, gd, ndim, sd, dims, pads, sync):
+        dims = [dims[k] for k in range(ndim)]
+        n = int(np.prod(dims))
+        at = [np.ctypeslib.as_array((C.c_double * n).from_address(p))
+              for p in (a, b, c, x, g, ga, gb, gc, gd)]
+        exp = oracle.adjoint(*[v.copy() for v in at[:5]], ndim, sd, dims)
+        for out, e in zip(at[5:], exp):
+            out[:] = e
+        return 0
+
+    def __getattr__(self, name):
+        if name == "tridDmtsvStridedBatchAdjoint":
+            return self._adjoint
+        raise AttributeError(name)
+
+
+def _oracle_solve(a, b, c, d, sd, u=None, inc=False, sync=1):
+    for t in (a, b, c, d):
+        assert t.is_contiguous() and t.shape == d.shape
+    dims = list(reversed(d.shape))
+    x = oracle_solve(*[t.numpy().ravel() for t in (a, b, c, d)], None, dims, sd)
+    d.copy_(torch.from_numpy(x.reshape(d.shape)))
+
+
+@pytest.fixture
+def on_host(monkeypatch):
+    monkeypatch.setattr(autograd, "lib", lambda: OracleLib())
+    monkeypatch.setattr(autograd, "solve", _oracle_solve)
+    monkeypatch.setattr(autograd, "_sync", lambda t: 1)
+
+
+def _transposed(t):
+    return t.detach().transpose(0, 2).contiguous().transpose(0, 2)
+
+
+def _sliced(t):
+    wide = torch.full((*t.shape[:-1], t.shape[-1] + 3), float("nan"), dtype=t.dtype)
+    wide[..., 2:-1] = t.detach()
+    return wide[..., 2:-1]
+
+
+def _expanded(t):
+    """One plane for all (its storage holds whole planes for every index)."""
+    room = torch.zeros_like(t)
+    room[0] = t.detach()[0]
+    return room[:1].expand(t.shape)
+
+
+@pytest.mark.parametrize("sd", [0, 1, 2])
+@pytest.mark.parametrize("make", [_transposed, _sliced, _expanded])
+def test_coefficients_of_any_strides(on_host, make, sd):
+    """Gradients with coefficients that are not contiguous are those with
+    contiguous copies of them."""
+    dims, shape = [6, 5, 4], (4, 5, 6)
+    t = [torch.from_numpy(v).reshape(shape) for v in dd_system(dims, sd, np.float64, seed=2)]
+    abc = [make(v) for v in t[:3]]
+    assert not any(v.is_contiguous() for v in abc)
+    g = torch.from_numpy(np.random.default_rng(1).uniform(-1, 1, shape))
+    got, exp = [], []
+    for out, coef in ((got, abc), (exp, [v.contiguous() for v in abc])):
+        leaves = [v.detach().requires_grad_(True) for v in (*coef, t[3])]
+        x = autograd.trid_solve(*leaves, sd)
+        out.append(x.detach())
+        out.extend(torch.autograd.grad(x, leaves, g))
+    for a, b in zip(got, exp):
+        assert torch.equal(a, b)

@@ -39,7 +39,9 @@ class TridSolve(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gx):
-        a, b, c, x = ctx.saved_tensors
+        # the adjoint takes dense arrays; the copies, like gx's, are dropped on
+        # torch's stream, behind the launch that reads them
+        a, b, c, x = (t.contiguous() for t in ctx.saved_tensors)
         gx = gx.contiguous()
         ga, gb, gc, gd = (torch.empty_like(x) for _ in range(4))
         dims = dims_of(x)
