@@ -4,6 +4,7 @@ is given."""
 from __future__ import annotations
 
 import ctypes as C
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -83,3 +84,21 @@ def test_coefficients_of_any_strides(on_host, make, sd):
         out.extend(torch.autograd.grad(x, leaves, g))
     for a, b in zip(got, exp):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("device,library,torch_stream,wait",
+                         [(0, 0, 0, 0), (0, 0, 7, 1), (0, 7, 0, 1), (0, 7, 7, 0),
+                          (1, 0, 0, 1), (1, 7, 7, 1)])
+def test_waits_unless_on_the_tensors_stream(monkeypatch, device, library, torch_stream, wait):
+    """Null streams have the same handle on every device: a call for a tensor
+    of another device than the current one waits whatever the handles."""
+    class Lib:
+        @staticmethod
+        def tridGetStream():
+            return library or None
+
+    monkeypatch.setattr(autograd, "lib", Lib)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "current_stream",
+                        lambda dev=None: SimpleNamespace(cuda_stream=torch_stream))
+    assert autograd._sync(SimpleNamespace(device=torch.device("cuda", device))) == wait

@@ -21,10 +21,14 @@ from .api import _iv, dims_of, solve
 def _sync(t) -> int:
     """0 where the library launches on the stream that torch works on for t's
     device: what follows there is ordered behind the call, and so is the reuse
-    of its temporaries; elsewhere 1, and the call waits for its results.
+    of its temporaries; elsewhere 1, and the call waits for its results.  The
+    library launches on the current device, and the null streams of all devices
+    have the same handle, so the device is compared as well.
     The waits kept the host from preparing the next launch: forward and
     backward of 1000 x 4000 FP32 took 176 us for 58 us of kernels."""
-    return int((lib().tridGetStream() or 0) != torch.cuda.current_stream(t.device).cuda_stream)
+    here = t.device.index == torch.cuda.current_device()
+    return int(not here or (lib().tridGetStream() or 0)
+               != torch.cuda.current_stream(t.device).cuda_stream)
 
 
 class TridSolve(torch.autograd.Function):
