@@ -46,7 +46,7 @@ def _oracle_solve(a, b, c, d, sd, u=None, inc=False, sync=1):
 def on_host(monkeypatch):
     monkeypatch.setattr(autograd, "lib", lambda: OracleLib())
     monkeypatch.setattr(autograd, "solve", _oracle_solve)
-    monkeypatch.setattr(autograd, "_sync", lambda t: 1)
+    monkeypatch.setattr(autograd, "_sync", lambda t: 0)
 
 
 def _transposed(t):
@@ -102,3 +102,32 @@ def test_waits_unless_on_the_tensors_stream(monkeypatch, device, library, torch_
     monkeypatch.setattr(torch.cuda, "current_stream",
                         lambda dev=None: SimpleNamespace(cuda_stream=torch_stream))
     assert autograd._sync(SimpleNamespace(device=torch.device("cuda", device))) == wait
+
+
+@pytest.mark.parametrize("wait", [0, 1])
+def test_other_streams_start_behind_torchs(on_host, monkeypatch, wait):
+    """Where the library launches on another stream, what torch has on its own
+    (the copies of the operands, an earlier call's results) is finished before
+    the launch; elsewhere nothing waits."""
+    log = []
+    stream = SimpleNamespace(synchronize=lambda: log.append("wait"))
+
+    class Lib(OracleLib):
+        def _adjoint(self, *args):
+            log.append(("adjoint", args[-1]))
+            return super()._adjoint(*args)
+
+    def solve(*args, sync):
+        log.append(("solve", sync))
+        _oracle_solve(*args)
+
+    monkeypatch.setattr(autograd, "lib", lambda: Lib())
+    monkeypatch.setattr(autograd, "solve", solve)
+    monkeypatch.setattr(autograd, "_sync", lambda t: wait)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev=None: stream)
+    dims = [6, 5]
+    t = [torch.from_numpy(v).reshape(5, 6).requires_grad_(True)
+         for v in dd_system(dims, 0, np.float64, seed=2)]
+    autograd.trid_solve(*t, 0).sum().backward()
+    start = ["wait"] * wait
+    assert log == start + [("solve", wait)] + start + [("adjoint", wait)]

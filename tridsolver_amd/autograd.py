@@ -31,12 +31,22 @@ def _sync(t) -> int:
                != torch.cuda.current_stream(t.device).cuda_stream)
 
 
+def _ordered(t) -> int:
+    """_sync(t) for a call that is made next.  Where it is 1, torch's stream is
+    waited for first: the library's stream is not ordered behind the copies of
+    the operands or behind an earlier call that did not wait."""
+    wait = _sync(t)
+    if wait:
+        torch.cuda.current_stream(t.device).synchronize()
+    return wait
+
+
 class TridSolve(torch.autograd.Function):
     @staticmethod
     def forward(ctx, a, b, c, d, solvedim: int):
         x = d.detach().clone().contiguous()
-        solve(a.detach().contiguous(), b.detach().contiguous(), c.detach().contiguous(), x,
-              solvedim, sync=_sync(x))
+        abc = [t.detach().contiguous() for t in (a, b, c)]
+        solve(*abc, x, solvedim, sync=_ordered(x))
         ctx.solvedim = solvedim
         ctx.save_for_backward(a, b, c, x)
         return x
@@ -53,11 +63,14 @@ class TridSolve(torch.autograd.Function):
               else lib().tridSmtsvStridedBatchAdjoint)
         _check(fn(a.data_ptr(), b.data_ptr(), c.data_ptr(), x.data_ptr(), gx.data_ptr(),
                   ga.data_ptr(), gb.data_ptr(), gc.data_ptr(), gd.data_ptr(), len(dims),
-                  ctx.solvedim, _iv(dims), _iv(dims), _sync(x)), "tridXmtsvStridedBatchAdjoint")
+                  ctx.solvedim, _iv(dims), _iv(dims), _ordered(x)), "tridXmtsvStridedBatchAdjoint")
         return ga, gb, gc, gd, None
 
 
 def trid_solve(a, b, c, d, solvedim: int):
+    """x = A^{-1} d along `solvedim`.  Where the library launches on torch's
+    stream the call does not wait; x is ordered on that stream, as the results
+    of torch's own operations are."""
     return TridSolve.apply(a, b, c, d, solvedim)
 
 
