@@ -116,6 +116,15 @@ def kernel_of_config(cfg: str, dtype: str, inc: int, coef: str, nx: int = 0):
         ys = nx // (64 * E) if nx and nx % (64 * E) == 0 else 0
         ys = ys if ys in (1, 2, 4) and ys < R // E else 0
         return f"k_adi_rhs_x<{T}, {R}, {int('cached' in fl)}, {int('cc' in fl)}, {ys}>"
+    m = re.search(r"rhs\+x\(lines,R(\d+)((?:,\w+)*)\)", cfg)
+    if m and nx >= 3:
+        # pieces per lane: those of a chunk's rows, or one less where the lines
+        # of a wave leave the last one empty
+        R, E = int(m.group(1)), (2 if T == "double" else 4)
+        np_max = -(-R // E)
+        lpw = min(64 // -(-(nx - 2) // R), np_max * 64 * E // nx)
+        pieces = max(np_max - 1, -(-lpw * nx // (64 * E)))
+        return f"k_adi_rhs_xl<{T}, {R}, {pieces}, {int('cached' in m.group(2).split(','))}>"
     return None
 
 
@@ -138,15 +147,14 @@ def traffic_from_profiles(key: str):
 
 def stage_config(desc: str, stage: str) -> str:
     """The configuration of one ADI stage from the plan's description
-    ("rhs+x(fused,R8)<double> x:... y:... z:...")."""
+    ("rhs+x(fused,R8)<double> x:... y:... z:...", and "step:rhs+x(lines,...)"
+    behind it where the fused stage runs the whole-line kernel)."""
     toks = desc.split()
-    pre = {"sweep_x": "x:", "sweep_y": "y:", "sweep_z_inc": "z:"}.get(stage)
-    if pre is None:
-        return toks[0] if toks else ""
+    pre = {"sweep_x": "x:", "sweep_y": "y:", "sweep_z_inc": "z:", "rhs_x_fused": "step:"}.get(stage)
     for t in toks:
-        if t.startswith(pre):
+        if pre and t.startswith(pre):
             return t
-    return ""
+    return toks[0] if toks and pre in (None, "step:") else ""
 
 
 def kernel_events(ta, pair):
@@ -213,11 +221,18 @@ def adi_workload(args, torch, np, api, ta):
     plan = AdiPlan(n, n, n, tdt, 1.0, 1)
     u0_dev = u.clone()
     pts = n ** 3
-    fused = "fused" in plan.describe()
+    desc = plan.describe()
     # algorithmic bytes per launch: rhs (+x when fused) reads u and writes du;
     # the x and y sweeps read and write du; the z sweep reads du and u and
     # writes u
-    if fused:
+    if "fused" not in desc and "lines" in desc:
+        # the right-hand side + x kernel of these grids has no stage number:
+        # whole steps are timed (u in, du out; du in, du out; du and u in, u
+        # out)
+        stages = (None,)
+        names = ("step",)
+        algo = [7 * wsize * pts]
+    elif "fused" in desc:
         stages = (4, 2, 3)
         names = ("rhs_x_fused", "sweep_y", "sweep_z_inc")
         algo = [2 * wsize * pts, 2 * wsize * pts, 3 * wsize * pts]
@@ -228,6 +243,13 @@ def adi_workload(args, torch, np, api, ta):
 
     def step(events=None):
         for i, g in enumerate(stages):
+            if g is None:
+                if events is not None:
+                    events[i][0].record()
+                plan.step(u, du, 1, sync=0)
+                if events is not None:
+                    events[i][1].record()
+                continue
             if events is not None:
                 kernel_events(ta, events[i])
             plan.stage(u, du, g)

@@ -53,9 +53,12 @@ EXTERN_C tridStatus_t tridAdiStep(tridAdiPlan_t plan, void *u, void *du,
  * 2 = y sweep, 3 = z sweep with u += , 4 = right-hand side fused with the x
  * sweep (for tests and per-kernel timing).  tridAdiStep uses 4, 2, 3 when
  * the plan supports the fused stage (tridAdiPlanDescribe says so) and u, du
- * are 16-byte aligned; else, and for some grids in place of stage 4, a kernel
- * of its own for stages 0 and 1 together (lines of at most 834 points, arrays
- * below 4 GiB, any alignment; "lines" in tridAdiPlanDescribe); else 0, 1, 2, 3. */
+ * are 16-byte aligned; stage 4 is then the kernel that the steps run (where
+ * tridAdiPlanDescribe ends in "step:", the whole-line one named there).  Else
+ * the steps run that whole-line kernel for stages 0 and 1 together where the
+ * grid fits it (lines of at most 834 points, arrays below 4 GiB, any
+ * alignment; "lines" in tridAdiPlanDescribe), which has no stage number; else
+ * 0, 1, 2, 3. */
 EXTERN_C tridStatus_t tridAdiStage(tridAdiPlan_t plan, void *u, void *du,
                                    int stage);
 

@@ -1071,8 +1071,8 @@ hipError_t launch_cc(const tridAdiPlan_st *p, int dir, T *d, T *u, hipStream_t s
 }
 
 // Stage 4 = fused RHS + x sweep (plans with fused_R > 0 only); kLinesStage
-// the whole-line one (lines_R > 0), which tridAdiStep takes where the fused
-// one does not apply.
+// the whole-line one (lines.R > 0), which the steps take where the fused one
+// does not apply or is the slower one (use_lines).
 constexpr int kLinesStage = 5;
 
 template <typename T>
@@ -1645,6 +1645,8 @@ EXTERN_C tridStatus_t tridAdiStage(tridAdiPlan_t p, void *u, void *du, int stage
   ensure_tuned(p, u, du);
   if (stage == 4 && !use_fused(p, u, du))
     return fail(TRID_STATUS_INVALID_VALUE, "this plan/layout has no fused RHS + x stage");
+  // stage 4 is the kernel that the steps run
+  if (stage == 4 && use_lines(p, u, du)) stage = kLinesStage;
   return stage_any(p, u, du, stage, current_stream());
 }
 
