@@ -297,9 +297,10 @@ inline std::string cfg_name(const PartCfg &c, size_t tsize) {
   if (c.kind == 2) {
     snprintf(buf, sizeof buf, "fallback<%s>", tsize == 8 ? "double" : "float");
   } else if (c.kind == 4) {
-    snprintf(buf, sizeof buf, "split<%s,o%d,R%d,L%d,spb%d%s>",
+    snprintf(buf, sizeof buf, "split<%s,o%d,R%d,L%d,spb%d%s%s%s>",
              tsize == 8 ? "double" : "float", c.order, c.R, c.R << c.cps_log2,
-             1 << c.spb_log2, c.vec >= 2 ? ",staged" : (c.vec ? ",vec" : ""));
+             1 << c.spb_log2, c.vec >= 2 ? ",staged" : (c.vec ? ",vec" : ""),
+             c.xcd ? ",xcd" : "", c.cp == kCached ? ",cached" : "");
   } else {
     snprintf(buf, sizeof buf, "part<%s,o%d,R%d,cps%d,spb%d%s%s%s>",
              tsize == 8 ? "double" : "float", c.order, c.R, chunk_count(c),

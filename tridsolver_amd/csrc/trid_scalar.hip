@@ -373,6 +373,9 @@ PartCfg autotune(int order, int vec, bool gvec, int idx32, bool dense, const T *
   return best;
 }
 
+// Strided systems of this many rows and more are solved in segments.
+constexpr int kSplitRows = 2048;
+
 template <typename T, int INC>
 tridStatus_t solve(const T *a, const int *a_pads, const T *b,
                    const int *b_pads, const T *c, const int *c_pads, T *d,
@@ -499,9 +502,10 @@ tridStatus_t solve(const T *a, const int *a_pads, const T *b,
     // `st` is being captured takes the untuned default (tuning synchronises
     // and times launches, which a capture cannot hold) and is tuned at its
     // first call outside a capture
-    // (a call with fixed scratch never tunes: tuning allocates)
+    // (a call with fixed scratch never tunes: tuning allocates; nor do the
+    // strided systems that are split below, whose layout is not a tuned one)
     bool have = false;
-    const bool tune = autotune_mode() == 1 && !fixed;
+    const bool tune = autotune_mode() == 1 && !fixed && !(order == 1 && D.N >= kSplitRows);
     tuned = tune;
     auto key = std::make_tuple((int)sizeof(T), INC, order, D.N, D.nsys,
                                vec * 4 + (int)gvec * 2 + (int)dense, D.sstr[3],
@@ -533,8 +537,11 @@ tridStatus_t solve(const T *a, const int *a_pads, const T *b,
   // i.e. 8- to 16-byte row runs (3-30 % of HBM bandwidth on MI355X), while
   // the split-line segments keep 64 systems side by side (about 69 % of its
   // 9 words per unknown, i.e. 38 % on the one-pass scale)
-  if (fc.kind == 0 && cfg.kind == 1 && order == 1 && D.N >= 2048) cfg.kind = 4;
-  if (cfg.kind == 4 && fc.kind != 4) cfg = split_cfg(order, vec, sizeof(T), D.nsys);
+  if (fc.kind == 0 && cfg.kind == 1 && order == 1 && D.N >= kSplitRows) cfg.kind = 4;
+  if (cfg.kind == 4 && fc.kind != 4) {
+    cfg = split_cfg(order, vec, sizeof(T), D.nsys);
+    tuned = false;  // (its policy too comes from the rule)
+  }
   if (cfg.kind == 4 && D.nsys > (1LL << 30))
     return fail(TRID_STATUS_INVALID_VALUE, "split-line solve: too many systems");
   if (cfg.kind == 4) {
