@@ -76,7 +76,8 @@ EXTERN_C tridStatus_t tridForceWideIndex(int on);
  * coefficients are not arrays: ADI plans, the variable-diffusivity ADI),
  * -1 (the default) = automatic: ordinary when the arrays of the call -- of
  * an ADI plan: u and du -- span at most 384 MiB (strided solves of one
- * launch along solvedim 0: 256 MiB), else 2 when d and u fit in 384 MiB,
+ * launch along solvedim 0 whose loads take whole cache lines: 256 MiB), else
+ * 2 when d and u fit in 384 MiB,
  * else non-temporal; with autotuning on, strided solves also time the other
  * policies.  Applies to
  * later strided solves and to ADI plans created afterwards; all policies

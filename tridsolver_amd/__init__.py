@@ -88,8 +88,9 @@ def force_cache_policy(policy: int) -> None:
     1 ordinary (arrays that fit the 256 MB last-level cache stay there for
     the next kernel or call), 2 non-temporal coefficient arrays with ordinary
     d and u, -1 automatic (ordinary up to 384 MiB of arrays per call or ADI
-    step, 256 MiB for a solvedim-0 solve of one launch, else 2 while d and u fit in 384 MiB, else 0).  All give bitwise
-    equal results."""
+    step, 256 MiB for a solvedim-0 solve of one launch whose loads take whole
+    cache lines, else 2 while d and u fit in 384 MiB, else 0).  All give
+    bitwise equal results."""
     _check(lib().tridForceCachePolicy(int(policy)), "tridForceCachePolicy")
 
 

@@ -71,7 +71,8 @@ inline hipError_t launch_kernel(F kernel, dim3 grid, dim3 block, std::uint32_t l
 // the previous one (or call) wrote there; else the mixed policy when d and u
 // fit (the coefficients stream past the cache and d stays in it);
 // non-temporal past that.  tridForceCachePolicy overrides the rule.  Solves
-// along solvedim 0 in one launch take the mixed policy from kMallBytes on.
+// along solvedim 0 in one launch whose loads take whole cache lines have the
+// mixed policy from kMallBytes on.
 constexpr size_t kMallBytes = 256ull << 20;
 constexpr size_t kMallFitBytes = 384ull << 20;
 int cache_policy(size_t bytes, size_t rhs_bytes = ~size_t(0));

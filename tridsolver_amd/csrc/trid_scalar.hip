@@ -559,10 +559,16 @@ tridStatus_t solve(const T *a, const int *a_pads, const T *b,
   // coefficients stream, so that they do not push d out of it.  Cached /
   // mixed, the same arrays again and others in turn: [256, 256, 160] FP64,
   // 320 MiB: 65 / 64 and 81 / 64 us, [300, 390, 170] FP32, 303 MiB: 63 / 62
-  // and 79 / 62, [200, 180, 250] FP64 Inc, 343 MiB: 74 / 68 and 84 / 79.
+  // and 79 / 62.  Only where each load of a wave takes whole cache lines
+  // (staged spans, or one 16-byte vector per chunk): lanes that come back to
+  // a line for their chunk's next rows read it again when it streams
+  // ([200, 180, 250] FP64 Inc with lines padded to 208, 357 MiB: 88 / 105 us;
+  // over 270..380 MiB 1.13 to 1.28 times, scalar rows 1.46 to 1.66 times).
   // Strided rows keep cached up to the rule's 384 MiB: [180, 200, 250] FP64,
   // 275 MiB, solvedim 1: 64 / 78 and 78 / 78
-  if (!tuned && order == 0 && cfg.kind == 1 && cfg.cp == kCached && footprint > kMallBytes)
+  const bool whole_loads = cfg.vec >= 2 || (cfg.vec == 1 && cfg.R * sizeof(T) == 16);
+  if (!tuned && order == 0 && cfg.kind == 1 && cfg.cp == kCached && footprint > kMallBytes &&
+      whole_loads)
     cfg.cp = kMixed;
   if (forced_cache_policy() >= 0) cfg.cp = forced_cache_policy();
   if (!idx32 || cfg.kind == 2) cfg.cp = kStream;
