@@ -309,7 +309,9 @@ tridStatus_t strided_adjoint(const T *a, const T *b, const T *c, const T *x, con
     // the strided batches' layout (most systems per work-group)
     const PartCfg s = strided_default(D.N, sizeof(T));
     if (s.kind == 1) cfg = s;
-    const PartCfg w = strided_wide(D.N, D.nsys, sizeof(T));
+    RowRuns rr;
+    rr.inc = true;  // (as many values per row in flight)
+    const PartCfg w = strided_wide(D.N, D.nsys, sizeof(T), rr);
     if (w.kind == 1) cfg = w;
   } else {
     const PartCfg s = adj_rows(D.N, aligned, dense);

@@ -312,7 +312,18 @@ inline std::string cfg_name(const PartCfg &c, size_t tsize) {
   return buf;
 }
 
-inline PartCfg strided_wide(int N, long long nsys, size_t tsize);
+// What the layouts of strided (solvedim >= 1) batches depend on besides the
+// lengths.
+struct RowRuns {
+  bool inc = false;    // the solution is added into u
+  bool cached = true;  // all arrays stay in the last-level cache (kMallFitBytes)
+  bool rhs = true;     // d and u do
+  bool small = true;   // at most 32 MiB of arrays
+  bool whole = false;  // row runs are whole cache lines (see row_runs)
+  bool far = true;     // rows of a system are 4 KiB and more apart,
+  bool alias = false;  // a multiple of 32 KiB
+};
+inline PartCfg strided_wide(int N, long long nsys, size_t tsize, RowRuns rr = {});
 
 inline std::vector<PartCfg> candidates(int order, int N, int vec, size_t tsize,
                                 bool dense, long long nsys, bool gvec = false) {
@@ -381,37 +392,96 @@ inline PartCfg strided_default(int N, size_t tsize) {
   return t;
 }
 
+// Row runs of a strided batch of n arrays (`ptrs`; 5 with u) of `bytes` bytes
+// in all: whole when every row of a run of systems starts on a 128-byte cache
+// line (bases, solve strides and the strides of the dimensions that do not
+// continue the run of the faster ones).
+inline RowRuns row_runs(const SysDesc &D, const void *const *ptrs, int n, size_t tsize,
+                        size_t bytes, size_t rhs_bytes) {
+  RowRuns rr;
+  rr.inc = n == 5;
+  rr.cached = bytes <= kMallFitBytes;
+  rr.rhs = rhs_bytes <= kMallFitBytes;
+  rr.small = bytes <= 32u << 20;
+  rr.whole = true;
+  rr.far = (unsigned long long)D.sstr[3] * tsize >= 4096;
+  rr.alias = (unsigned long long)D.sstr[3] * tsize % 32768 == 0;
+  for (int t = 0; t < n; t++) {
+    rr.whole &= reinterpret_cast<uintptr_t>(ptrs[t]) % 128 == 0 && D.sstr[t] * tsize % 128 == 0;
+    long long run = 1;
+    for (int k = 0; k < D.nother; k++) {
+      if (D.ostr[t][k] == run) run *= D.osize[k];
+      else rr.whole &= D.ostr[t][k] * tsize % 128 == 0;
+    }
+  }
+  return rr;
+}
+
 // Layout of strided batches of at least 64 work-groups, where all of the chip
-// is at work (smaller ones keep strided_default or the heuristic):
-//   * the XCD-contiguous order at every length: a work-group's row runs end
-//     inside cache lines that its neighbours' begin in, and neighbours then
-//     share an L2.  Runs of whole lines lose nothing ([256, 256, 256] FP64
-//     115 -> 112 us, [256, 128, 300] FP32 44.5 -> 45), others gain
-//     ([149, 100, 300] FP32 27 -> 19, [149, 220, 244] FP64 91 -> 71).
-//   * the chunk count cut to the rows where that drops a quarter of the
-//     power of two or more (150 rows: 20 chunks of 8, not 32), which makes
-//     room for twice the systems side by side ([150, 150, 150] FP64 35 -> 32
-//     us, [300, 333, 150] FP32 81 -> 74); nearer the power of two the extra
-//     idle lanes cost nothing (220 rows: 28 chunks 77, 32 chunks 71 us).
-//   * FP64, 257..512 rows: 8 systems in 256 threads, four work-groups per CU,
-//     against 16 in 512 ([149, 450, 119] 89 -> 80 us); 513..768 rows: 8-row
-//     chunks, which leave fewer rows idle ([256, 600, 52] 95 -> 79 us).
-//   * FP32 up to 128 rows: 16-row chunks ([149, 128, 300] 26.7 -> 26.3 us,
-//     [256, 70, 300] 25 -> 22); 385..512 rows: 16 systems in 512 threads
-//     ([149, 450, 178] 71 -> 68).
-// Microseconds on MI355X, batches cycled through several sets of arrays.
+// is at work (smaller ones keep strided_default or the heuristic).  Ratios are
+// times against those layouts, geometric means [extremes] over widths 200 to
+// 512, three sizes and both strided dimensions on MI355X, inputs in turn.
+//   * the XCD-contiguous order where row runs end inside cache lines: the
+//     neighbours' begin there, and neighbours then share an L2 ([149, 100,
+//     300] FP32 27 -> 19 us, [149, 220, 244] FP64 91 -> 71).  Whole-line runs
+//     share none, and FP64 up to 128 rows is faster in the plain order (XCD
+//     1.03 [0.97, 1.15]); 129..256 rows too while rows are less than a page
+//     apart (1.04 to 1.07; 4 KiB and more 0.96 [0.82, 1.07]), and 257..512
+//     rows past the cache (1.00 [0.90, 1.07]).
+//   * FP64, 129..256 rows: 16 systems of 8-row chunks (0.86 to 0.92), up to
+//     192 rows of 16-row chunks unless Inc (0.95 of the former).  Chunk counts
+//     cut to the rows, with 32 systems side by side (150 rows: 20 chunks, not
+//     32), only in batches of at most 32 MiB and past the cache (0.77, against
+//     0.87; Inc where d and u are past it too, 0.87 against 0.92), and not for
+//     whole-line runs (1.08).
+//   * FP64, 257..512 rows: cached, 8 systems in 256 threads, four work-groups
+//     per CU (Inc 0.82, else 0.88).  Past the cache their 64-byte runs are
+//     fetched twice (1.01 to 1.27): 16 systems there, as where more than 384
+//     rows 32 KiB apart meet in the cache ([64, 256, 512], solvedim 2: 1.16);
+//     Inc with 8-row chunks (0.84 to 0.92: half the live rows).
+//   * FP64, 513..768 rows: 8-row chunks cut to the rows, cached 0.84, Inc
+//     0.82 to 0.86 at any size; else past the cache 1.04 to 1.26.
+//   * FP32 up to 128 rows: 64 systems of 16-row chunks (0.78 to 0.94), but not
+//     whole-line runs of up to 64 rows (1.06) or of rows 32 KiB apart (1.04).
+//   * FP32, 129..256 rows: chunks cut to the rows for Inc (0.92 to 0.98), for
+//     whole-line runs past the cache (0.98), and where nearly half of them go
+//     (140 rows: 18 of 32 chunks, 0.95; 150 rows: 20 of 32, 1.03).
+//   * FP32, 257..384 rows: cut for Inc (0.78 to 0.91), cached (0.90) and
+//     whole-line (0.92) batches; others past the cache 1.03 [0.95, 1.12].
+//   * FP32, 385..512 rows, cached: 16 systems in 512 threads (385..448 rows
+//     0.90; 449..512 rows 0.96, Inc 0.87, whole-line 1.01); past the cache
+//     1.1 to 1.4.
+//   * FP32, 513..2048 rows: cut where cached (0.9) and, for Inc, where d and u
+//     are (0.94); past the cache 1.03 to 1.09.
 // Returns kind 0 when the rule does not apply.
-inline PartCfg strided_wide(int N, long long nsys, size_t tsize) {
+inline PartCfg strided_wide(int N, long long nsys, size_t tsize, RowRuns rr) {
   PartCfg c;
   c.kind = 0;
   if (N > 2048) return c;
+  const bool f64 = tsize == 8;
   int R, spb;
-  if (tsize == 8) {
-    R = N <= 256 || (N > 512 && N <= 768) ? 8 : 16;
-    spb = N <= 256 ? 512 / std::max(8, 1 << ilog2((N + 7) / 8)) : N <= 1024 ? 8 : 4;
+  bool cut = false;  // chunk count cut to the rows
+  if (f64) {
+    const bool out = N > 256 && N <= 512 && ((rr.alias && N > 384) || !rr.cached);
+    if (N > 512 && !rr.cached && !(rr.inc && N <= 768)) return c;
+    R = N <= 256 || (N > 512 && N <= 768) || (out && rr.inc && !rr.alias) ? 8 : 16;
+    spb = N <= 256 ? 512 / std::max(8, 1 << ilog2((N + 7) / 8))
+                   : out ? 16 : N <= 1024 ? 8 : 4;
+    cut = N <= 256 ? !rr.whole && (rr.small || (!rr.cached && !(rr.inc && rr.rhs)))
+                   : N > 512 && N <= 768;
+    if (N > 128 && N <= 192 && !cut && !rr.inc) R = 16;
   } else {
+    if (N <= 128 ? rr.whole && (N <= 64 || rr.alias)
+                 : N > 384 && N <= 512 &&
+                       (!rr.cached || rr.alias || (N > 448 && rr.whole && !rr.inc)))
+      return c;
     R = N > 128 && N <= 256 ? 8 : 16;
     spb = N <= 128 ? 64 : N <= 384 ? 32 : N <= 1024 ? 16 : 8;
+    cut = N <= 128 || (N > 384 && N <= 512) ? false
+          : N <= 256 ? rr.inc || (rr.cached ? !rr.whole && N <= 144 : rr.whole)
+          : N <= 384 ? rr.inc || rr.cached || rr.whole
+                     : rr.cached || (rr.inc && rr.rhs);
+    if (N > 128 && !(N > 384 && N <= 512) && !cut) return c;
   }
   const int chunks = (N + R - 1) / R, cps = 1 << ilog2(chunks);
   PartCfg t = make_cfg(1, R, N, 0, 512);
@@ -422,13 +492,19 @@ inline PartCfg strided_wide(int N, long long nsys, size_t tsize) {
     const int m = side >= kWave ? 1 : kWave / side;
     return (chunks + m - 1) / m * m;
   };
-  if (tsize == 8 && N <= 256 && cps >= 16 && 4 * trim(32) <= 3 * cps) {
-    t.spb_log2 = 5;
-    t.cps_any = trim(32);
-  } else if (4 * trim(spb) <= 3 * cps && (tsize == 4 ? N > 128 : N > 512 && N <= 768)) {
-    t.cps_any = trim(spb);
+  // (nearer the power of two than three quarters the idle lanes cost nothing:
+  // 220 rows: 28 chunks 77, 32 chunks 71 us)
+  if (cut) {
+    const int side = f64 && N <= 256 ? 32 : spb;
+    if (cps >= 16 && 4 * trim(side) <= 3 * cps) {
+      t.spb_log2 = ilog2(side);
+      t.cps_any = trim(side);
+    }
   }
-  t.xcd = 1;
+  t.xcd = !(f64 && rr.whole &&
+            (N <= 128 || (N <= 256 ? !rr.far
+                                   : N <= 512 && ((rr.alias && N > 384) ||
+                                                  (!rr.cached && !rr.inc)))));
   if (!cfg_valid(t, N, tsize) || (nsys >> t.spb_log2) < 64) return c;
   return t;
 }

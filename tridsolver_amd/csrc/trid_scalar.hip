@@ -139,12 +139,13 @@ inline long long round4(long long v) { return (v + 3) & ~3LL; }
 // the strided default for solvedim >= 1, wave staging where it applies and
 // the chunk length that pads a solvedim-0 system least.
 template <typename T>
-PartCfg default_cfg(int order, const SysDesc &D, int vec, bool gvec, bool dense) {
+PartCfg default_cfg(int order, const SysDesc &D, int vec, bool gvec, bool dense,
+                    RowRuns rr = {}) {
   PartCfg cfg = heuristic(order, D.N, vec, sizeof(T));
   if (order == 1 && cfg.kind == 1) {
     const PartCfg s = strided_default(D.N, sizeof(T));
     if (s.kind == 1) cfg = s;
-    const PartCfg w = strided_wide(D.N, D.nsys, sizeof(T));
+    const PartCfg w = strided_wide(D.N, D.nsys, sizeof(T), rr);
     if (w.kind == 1) cfg = w;
   }
   // staging pays when a chunk is more than one 16-byte vector
@@ -460,6 +461,7 @@ tridStatus_t solve(const T *a, const int *a_pads, const T *b,
     if (t == 4 && !INC) break;
     for (int k = 0; k < ndim; k++) dense &= pads[t][k] == dims[k];
   }
+  const RowRuns rr = row_runs(D, ptrs, INC ? 5 : 4, sizeof(T), footprint, rhs_bytes);
   hipStream_t st = current_stream();
   PartCfg cfg;
   bool tuned = false;  // cfg (and its cache policy) from the autotuner
@@ -527,7 +529,7 @@ tridStatus_t solve(const T *a, const int *a_pads, const T *b,
       have = true;
     }
     if (!have) {
-      cfg = default_cfg<T>(order, D, vec, gvec, dense);
+      cfg = default_cfg<T>(order, D, vec, gvec, dense, rr);
       tuned = false;
     }
   }
