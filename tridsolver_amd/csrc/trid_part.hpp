@@ -137,14 +137,15 @@ __device__ __forceinline__ void seg_merge(Row<T> &f, Row<T> &l, const Row<T> &fb
 // the work-group's systems are segments of L = SysDesc::N rows of longer
 // systems of N rows each, P per system, the last one possibly shorter.  Each
 // segment's two merged reduced rows go to rows 2p and 2p+1 of its system's
-// reduced system of 2P rows (b = 1), at element 2P * qs + row of ra, rb, rc,
-// rd: reduced systems are contiguous whatever the order of the long ones.
+// reduced system of 2P rows (b = 1), at element qs * rs_sys + row * rs_row of
+// ra, rb, rc, rd (contiguous systems, or in the long systems' order).
 //   segment item q -> (system qs, segment p): ORDER 0: p = q % P, qs = q / P;
 //   ORDER 1: qs = q % nsys, p = q / nsys.
 template <typename T>
 struct SegOut {
   T *ra = nullptr, *rb = nullptr, *rc = nullptr, *rd = nullptr;
   long long nsys = 0;
+  long long rs_row = 1, rs_sys = 0;
   int P = 1, N = 0;
 };
 
@@ -1087,10 +1088,10 @@ __device__ __forceinline__ void part_block(const Coef &coef, T *__restrict__ Dd,
   }
   if constexpr (MODE == 2) {
     if (active && (row0 == 0 || row0 + R == N)) {
-      const T *x = so.rd + (2LL * so.P * seg_qs + 2LL * seg_p);
-      if (row0 == 0 && seg_p > 0) d[0] -= *at(coef.A, off[0]) * x[-1];
+      const T *x = so.rd + (so.rs_sys * seg_qs + 2LL * seg_p * so.rs_row);
+      if (row0 == 0 && seg_p > 0) d[0] -= *at(coef.A, off[0]) * x[-so.rs_row];
       if (row0 + R == N && seg_p + 1 < so.P)
-        d[R - 1] -= *at(coef.C, off[2] + (I)(N - 1) * s2) * x[2];
+        d[R - 1] -= *at(coef.C, off[2] + (I)(N - 1) * s2) * x[2 * so.rs_row];
     }
   }
   if constexpr (MODE == 1) {
@@ -1156,15 +1157,15 @@ __device__ __forceinline__ void part_block(const Coef &coef, T *__restrict__ Dd,
     if (k == 0 && active) {
       const T as = seg_p > 0 ? *at(coef.A, off[0]) : T(0);
       const T ce = seg_p + 1 < so.P ? *at(coef.C, off[2] + (I)(N - 1) * s2) : T(0);
-      const long long i0 = 2LL * so.P * seg_qs + 2LL * seg_p;
+      const long long i0 = so.rs_sys * seg_qs + 2LL * seg_p * so.rs_row, i1 = i0 + so.rs_row;
       so.ra[i0] = f.a * as;
       so.rb[i0] = T(1);
       so.rc[i0] = f.c;
       so.rd[i0] = f.d;
-      so.ra[i0 + 1] = l.a;
-      so.rb[i0 + 1] = T(1);
-      so.rc[i0 + 1] = l.c * ce;
-      so.rd[i0 + 1] = l.d;
+      so.ra[i1] = l.a;
+      so.rb[i1] = T(1);
+      so.rc[i1] = l.c * ce;
+      so.rd[i1] = l.d;
     }
     return;
   }

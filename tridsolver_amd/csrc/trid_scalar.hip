@@ -166,20 +166,22 @@ PartCfg default_cfg(int order, const SysDesc &D, int vec, bool gvec, bool dense,
   return pick_rows(cfg, D.N, gvec, dense, sizeof(T));
 }
 
-// Configuration of the reduced systems (2P contiguous rows each, ns of them):
-// one launch, or a split-line solve of their own past one work-group.
+// Configuration of the reduced systems (2P rows each), contiguous (order 0) or
+// in the order of strided long ones (order 1): one launch, or a split-line
+// solve of their own past one work-group.
 template <typename T>
-PartCfg reduced_cfg(const SysDesc &Dr) {
-  const int vec = (Dr.N * (int)sizeof(T)) % 16 == 0;
-  PartCfg c = default_cfg<T>(0, Dr, vec, true, true);
+PartCfg reduced_cfg(int order, const SysDesc &Dr) {
+  const int vec = order == 0 && (Dr.N * (int)sizeof(T)) % 16 == 0;
+  PartCfg c = order == 0 ? default_cfg<T>(0, Dr, vec, true, true)
+                         : heuristic(1, Dr.N, 0, sizeof(T));
   if (c.kind != 1) {
-    c = split_cfg(0, vec, sizeof(T), Dr.nsys);
+    c = split_cfg(order, vec, sizeof(T), Dr.nsys);
     c.vec = split_vec(c, Dr.N, vec, true, sizeof(T));
   }
   return c;
 }
 
-SysDesc reduced_desc(int P, long long ns) {
+SysDesc reduced_desc(int order, int P, long long ns) {
   SysDesc D;
   memset(&D, 0, sizeof D);
   D.N = 2 * P;
@@ -187,11 +189,25 @@ SysDesc reduced_desc(int P, long long ns) {
   D.nother = 1;
   D.osize[0] = (int)ns;
   for (int t = 0; t < 5; t++) {
-    D.sstr[t] = 1;
-    D.ostr[t][0] = 2LL * P;
+    D.sstr[t] = order == 0 ? 1 : ns;
+    D.ostr[t][0] = order == 0 ? 2LL * P : 1;
   }
   D.small_index = !wide_index();
   return D;
+}
+
+// Order of the reduced systems of ns long ones of P segments each.  Strided
+// ones: contiguous while they are few and short enough for one launch (one
+// launch of few work-groups took 61 us of 162 at 48 x 150000 rows FP64; 700 x
+// 2048 FP32 18.2 against 19.4 us).  1024 systems and more fill the chip in the
+// long systems' order, whose lanes read and write whole lines where contiguous
+// ones scatter 2P apart (4096 x 8192 rows FP64 402 against 414 us, 333 x 4096
+// x 30 638 against 701); so do nested segments (64 x 2^19 rows 427 against
+// 464).
+template <typename T>
+int reduced_order(int order, int P, long long ns) {
+  if (order == 0) return 0;
+  return ns < 1024 && reduced_cfg<T>(0, reduced_desc(0, P, ns)).kind == 1 ? 0 : 1;
 }
 
 // Workspace (elements) of a split-line solve, including its recursive
@@ -201,7 +217,8 @@ long long split_ws_elems(const PartCfg &cfg, int N, long long nsys) {
   const long long L = (long long)cfg.R << cfg.cps_log2;
   const long long P = (N + L - 1) / L;
   long long need = 4 * round4(2 * P * nsys);
-  const PartCfg cr = reduced_cfg<T>(reduced_desc((int)P, nsys));
+  const int ro = reduced_order<T>(cfg.order, (int)P, nsys);
+  const PartCfg cr = reduced_cfg<T>(ro, reduced_desc(ro, (int)P, nsys));
   if (cr.kind != 1) need += split_ws_elems<T>(cr, (int)(2 * P), nsys);
   return need;
 }
@@ -223,6 +240,9 @@ hipError_t split_solve(const PartCfg &cfg, const T *a, const T *b, const T *c, T
   so.nsys = ns;
   so.P = P;
   so.N = N;
+  const int ro = reduced_order<T>(order, P, ns);
+  so.rs_row = ro == 0 ? 1 : ns;
+  so.rs_sys = ro == 0 ? 2LL * P : 1;
 
   // the segments as one batch: the segment index is one more non-solve
   // dimension (fastest for ORDER 0, so that a system's segments are adjacent
@@ -243,13 +263,16 @@ hipError_t split_solve(const PartCfg &cfg, const T *a, const T *b, const T *c, T
   cs.kind = 1;
 
   const CoefArrays<T> cf{a, b, c};
+  // (one segment per system is the whole of it: no couplings; 1 x 4000 rows
+  // FP64 21 us for the three launches)
+  if (P == 1) return launch_seg<T, 2, INC>(cs, cf, d, u, Ds, so, st);
   // 1. segment reduction
   hipError_t e = launch_seg<T, 1, 0>(cs, cf, d, nullptr, Ds, so, st);
   if (e != hipSuccess) return e;
 
   // 2. reduced systems
-  const SysDesc Dr = reduced_desc(P, ns);
-  PartCfg cr = reduced_cfg<T>(Dr);
+  const SysDesc Dr = reduced_desc(ro, P, ns);
+  PartCfg cr = reduced_cfg<T>(ro, Dr);
   cr.idx32 = (unsigned long long)n2 * sizeof(T) < (1ULL << 32) && !wide_index();
   cr.cp = cr.idx32 ? kCached : kStream;
   if (cr.kind == 1)
@@ -548,10 +571,13 @@ tridStatus_t solve(const T *a, const int *a_pads, const T *b,
     return fail(TRID_STATUS_INVALID_VALUE, "split-line solve: too many systems");
   if (cfg.kind == 4) {
     cfg.vec = split_vec(cfg, D.N, vec, gvec, sizeof(T));
-    // strided row runs end inside cache lines that the next work-group's
-    // begin in: neighbours share an XCD's L2 ([300, 3000, 10] FP32, ordinary
-    // loads: 95 -> 79 us); whole spans (ORDER 0) share none
-    cfg.xcd = order == 1;
+    // strided row runs that end inside cache lines, where the next
+    // work-group's begin: neighbours share an XCD's L2 ([300, 3000, 10] FP32,
+    // ordinary loads: 95 -> 79 us).  Runs of whole lines share none (4096 x
+    // 8192 rows FP64 402, 430 in the XCD order) and take it only where few
+    // systems' segments stay in the cache from one pass to the next (64 x
+    // 131072 FP32 65 -> 56); whole spans (ORDER 0) share none
+    cfg.xcd = order == 1 && (!rr.whole || (footprint < kMallBytes && D.nsys < 256));
   }
   cfg.idx32 = idx32;
   // cache policy: the tuned one, else the footprint rule; a forced policy
@@ -572,11 +598,14 @@ tridStatus_t solve(const T *a, const int *a_pads, const T *b,
   if (!tuned && order == 0 && cfg.kind == 1 && cfg.cp == kCached && footprint > kMallBytes &&
       whole_loads)
     cfg.cp = kMixed;
+  if (cfg.kind == 4 && rr.whole && footprint >= kMallBytes) cfg.cp = kStream;
   if (forced_cache_policy() >= 0) cfg.cp = forced_cache_policy();
   if (!idx32 || cfg.kind == 2) cfg.cp = kStream;
   // split-line: no mixed form, and ORDER 0 streams (2 x 2^22 rows FP64 122
   // against 132 us with ordinary loads; ORDER 1 [51, 7548, 19] FP32 103
-  // against 77)
+  // against 77); so do whole-line runs from the cache's own 256 MiB on, whose
+  // second pass finds little of the first (4096 x 2048 rows FP64 106 against
+  // 118 us with ordinary loads, 512 x 4096 x 4 113 against 120)
   if (cfg.kind == 4 && (cfg.cp != kCached || order == 0)) cfg.cp = kStream;
   set_last_config(cfg_name(cfg, sizeof(T)));
   // launch events (tridSetLaunchEvents) time single-kernel solves only
