@@ -41,8 +41,8 @@ EXTERN_C tridStatus_t tridSetLaunchEvents(void *start, void *stop);
 EXTERN_C const char *tridGetLastError(void);
 EXTERN_C const char *tridGetStatusString(tridStatus_t status);
 
-/* Describes the kernel configuration the last strided-batch call on this
- * thread used, e.g. "part<double,o0,R8,cps32,spb8>" (for reports and tests). */
+/* Describes the kernel configuration the last strided-batch call (or
+ * variable-diffusivity sweep) on this thread used, e.g. "part<double,o0,R8,cps32,spb8>" (for reports and tests). */
 EXTERN_C const char *tridGetLastConfig(void);
 
 /* Forces the next strided-batch calls onto one kernel configuration

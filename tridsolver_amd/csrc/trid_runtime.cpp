@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
@@ -26,6 +27,8 @@ std::mutex g_mu;
 ForcedConfig g_forced;
 thread_local std::string t_error;
 thread_local std::string t_config;
+thread_local std::string (*t_config_text)(const void *) = nullptr;  // not yet in t_config
+alignas(8) thread_local unsigned char t_config_data[64];
 thread_local LaunchEvents t_events;
 
 struct DevWs {
@@ -55,7 +58,15 @@ tridStatus_t fail(tridStatus_t st, const std::string &msg) {
 
 void clear_error() { t_error.clear(); }
 
-void set_last_config(const std::string &cfg) { t_config = cfg; }
+void set_last_config(const std::string &cfg) {
+  t_config_text = nullptr;
+  t_config = cfg;
+}
+
+void set_last_config(std::string (*text)(const void *), const void *data, size_t bytes) {
+  std::memcpy(t_config_data, data, std::min(bytes, sizeof t_config_data));
+  t_config_text = text;
+}
 
 tridStatus_t check_hip(hipError_t e, const char *what) {
   if (e == hipSuccess) return TRID_STATUS_SUCCESS;
@@ -189,7 +200,10 @@ EXTERN_C tridStatus_t tridSetAutotune(int mode) {
 
 EXTERN_C const char *tridGetLastError(void) { return t_error.c_str(); }
 
-EXTERN_C const char *tridGetLastConfig(void) { return t_config.c_str(); }
+EXTERN_C const char *tridGetLastConfig(void) {
+  if (t_config_text) set_last_config(t_config_text(t_config_data));
+  return t_config.c_str();
+}
 
 EXTERN_C const char *tridGetStatusString(tridStatus_t s) {
   switch (s) {

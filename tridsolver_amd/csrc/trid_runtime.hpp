@@ -19,6 +19,9 @@ hipStream_t current_stream();
 tridStatus_t fail(tridStatus_t st, const std::string &msg);
 void clear_error();
 void set_last_config(const std::string &cfg);
+// The same with the text made when it is asked for, from a copy of `bytes`
+// (at most 64) bytes: calls of a few microseconds do not pay for it.
+void set_last_config(std::string (*text)(const void *), const void *data, std::size_t bytes);
 
 // Maps a HIP error to a status (and records it); hipSuccess -> SUCCESS.
 tridStatus_t check_hip(hipError_t e, const char *what);

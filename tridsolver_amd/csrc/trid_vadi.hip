@@ -571,29 +571,62 @@ int vadi_policy(const Grid &g) {
   return p == kMixed ? kCached : p;  // no coefficient arrays: d and u cached
 }
 
+// Layout of the kappa sweep along `axis` (kind 1 unless the lines are too
+// long).
+PartCfg vadi_layout(const Grid &g, int axis, const SysDesc &D, const double *K, const double *d) {
+  const int order = axis == 0 ? 0 : 1;
+  PartCfg cfg = heuristic(order, D.N, 0, sizeof(double));
+  if (cfg.kind != 1) return cfg;
+  // Grids of up to 2^21 points leave the chip part idle; other chunks and
+  // work-groups put more of them on it (one sweep, heuristic -> this).
+  //   x sweeps, 4-row chunks: the loss and its gradient take these past the
+  //     576 points of the whole-line kernel (600 x 50 x 50 18.5 -> 15.8 us,
+  //     1000 x 40 x 40 18.5 -> 13.3), tridVadiSweep always (96^3 11.7 -> 8.8).
+  //   y and z sweeps of lines up to 64 points, 4-row chunks of 8 systems where
+  //     the heuristic has at most 128 work-groups (33^3 6.5 -> 4.7, 64^3 6.7 ->
+  //     5.9, loss and gradient of 256 x 32 x 32 293 -> 239; more of them lose to
+  //     its longer row runs: 20 x 20 x 1000 6.3 -> 8.6, 256 x 128 x 64 10.4 ->
+  //     19).
+  //   65..128 points, 8-row chunks of 16 systems where the heuristic's 32
+  //     leave the CUs uneven, more than one work-group each, and the 128-byte
+  //     runs are whole cache lines (96^3 9.1 -> 7.9, 128^3 10.8 -> 10.4; off
+  //     the line 113^3 13.2 -> 17.8; one each 80^3 6.9 -> 7.1).
+  //   257..512 points, 16 systems, not 8, for whole lines or at most 256
+  //     work-groups (64 x 300 x 64 16.4 -> 11.8, 30 x 100 x 400 14.9 -> 12.8;
+  //     neither 100 x 50 x 300 19.8 -> 21.0).
+  if (g.n <= 1LL << 21 && order == 0) {
+    const PartCfg t = make_cfg(0, 4, D.N, 0, 256);
+    if (cfg_valid(t, D.N)) cfg = t;
+  } else if (g.n <= 1LL << 21) {
+    const void *ptrs[4] = {K, K, K, d};
+    const bool whole = row_runs(D, ptrs, 4, sizeof(double), 0, 0).whole;
+    const long long wgs = (D.nsys + (1 << cfg.spb_log2) - 1) >> cfg.spb_log2;
+    PartCfg t = make_cfg(1, D.N <= 64 ? 4 : 8, D.N, 0, 256);
+    t.spb_log2 = D.N <= 64 ? 3 : 4;
+    const bool take = D.N <= 64    ? wgs <= 128
+                      : D.N <= 128 ? whole && wgs > 256
+                                   : D.N > 256 && (whole || D.nsys <= 256 * 16);
+    if (take && cfg_valid(t, D.N)) cfg = t;
+  }
+  cfg.vec = 0;
+  cfg.idx32 = (unsigned long long)g.n * 8 < (1ULL << 32) && !wide_index();
+  cfg.cp = cfg.idx32 ? vadi_policy(g) : kStream;
+  return cfg;
+}
+
+std::string sweep_text(const void *cfg) {
+  return cfg_name(*static_cast<const PartCfg *>(cfg), sizeof(double));
+}
+
 // Generic kappa sweep along `axis` (partitioned Thomas, scalar loads):
 // non-inc: out (default d) = A^{-1} d or A^{-T} d; inc: out (default u) =
 // u + A^{-1} d.
 tridStatus_t vadi_sweep(const double *K, double *d, double *u, double *out, const Grid &g,
                         int axis, double lam, int transpose, int inc, hipStream_t st) {
   const SysDesc D = line_desc(g, axis);
-  const int order = axis == 0 ? 0 : 1;
-  PartCfg cfg = heuristic(order, D.N, 0, sizeof(double));
+  const PartCfg cfg = vadi_layout(g, axis, D, K, d);
   if (cfg.kind != 1) return fail(TRID_STATUS_INVALID_VALUE, "vadi: grid too long along an axis");
-  // grids of up to 2^21 points leave the chip part idle: shorter chunks and
-  // smaller work-groups put more of them on it.  Loss and gradient of 8
-  // steps, heuristic -> this: y and z sweeps of 40^3 616 -> 553 us (4-row
-  // chunks, 8 systems), 64^3 585 -> 507, 96^3 1044 -> 999 (8 rows, 16
-  // systems), 128^3 1203 -> 1182; x sweeps (4 rows) 96^3 1044 -> 995, 113^3
-  // 1366 -> 1268
-  if (g.n <= 1LL << 21) {
-    PartCfg t = make_cfg(order, order == 0 || D.N <= 64 ? 4 : 8, D.N, 0, 256);
-    if (order == 1) t.spb_log2 = D.N <= 64 ? 3 : 4;
-    if (cfg_valid(t, D.N)) cfg = t;
-  }
-  cfg.vec = 0;
-  cfg.idx32 = (unsigned long long)g.n * 8 < (1ULL << 32) && !wide_index();
-  cfg.cp = cfg.idx32 ? vadi_policy(g) : kStream;
+  set_last_config(&sweep_text, &cfg, sizeof cfg);
   const CoefKappa<double> cf{K, lam, transpose};
   hipError_t e = inc ? launch_part<double, 1>(cfg, cf, d, u, D, st, out)
                      : launch_part<double, 0>(cfg, cf, d, u, D, st, out);
