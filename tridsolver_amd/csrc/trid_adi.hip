@@ -865,8 +865,10 @@ bool cc_pair_fits(const tridAdiPlan_st *p, int R, int cps) {
 //     per lane (128^3 FP64 z 16.4 -> 11.6 us with 8-row chunks; 200 x 150 x
 //     180 FP32 z -3.2 us of 46).  Wide rows carry the long lines: 512^3 FP32
 //     z 302 -> 185 us, 300^3 -25 of 203.
-//   rows: 8 up to 128-row lines (FP64 pairs 16: 256 x 256 x 128 z -2.7 us),
-//     16 up to 256, else 32.
+//   rows: 8 up to 128-row lines (FP64 pairs 16: 256 x 256 x 128 z -2.7 us; FP64
+//     lines past 96 rows 16 too where there are more than one work-group per
+//     CU: 333 x 100 x 100 y 14.6 -> 11.4, z 21.9 -> 17.3 us; 99^3, fewer, y 7.6
+//     against 8.3; 300 x 70 x 100, y 8.9 against 9.5), 16 up to 256, else 32.
 //   xcd: y always (512^3 FP64 -104 us of 1708, 200 x 150 x 180 FP32 -1.2 of
 //     46: the lines of a work-group and of the next share row ends); z while
 //     the arrays stay in the last-level cache (256^3 FP64 -9 us of 170; past
@@ -877,7 +879,8 @@ struct CCChoice {
 bool cc_default(const tridAdiPlan_st *p, int dir, CCChoice *c) {
   const SysDesc &D = p->desc[dir];
   const bool wide = D.osize[0] % 2 == 0 && D.nsys >= 256LL * 2 * kWave;
-  c->R = D.N > 256 ? 32 : (D.N > 128 || (p->dbl && wide) ? 16 : 8);
+  const bool many = D.N > 96 && D.nsys > 256LL * kWave;
+  c->R = D.N > 256 ? 32 : (D.N > 128 || (p->dbl && (wide || many)) ? 16 : 8);
   if (!cc_rows_ok(D.N, c->R, &c->cps)) return false;
   c->pair = wide && cc_pair_fits(p, c->R, c->cps);
   c->xcd = dir == 1 || p->cp == kCached;
