@@ -1155,12 +1155,12 @@ __device__ __forceinline__ void blk2_tw_block(const BlkArgs<T> &g, long long blo
 }
 
 template <typename T, int M, int TRANS>
-__global__ void __launch_bounds__(256, blk2_min_waves(M)) k_blk2_tw(BlkArgs<T> g) {
+__global__ void __launch_bounds__(256, blk2_min_waves(M)) k_blk2_tw(BlkArgs<T> g, int xcd) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  // XCD-contiguous order (as k_part): a wave's run of blocks ends inside a
-  // cache line that the next one's begins in
+  // XCD-contiguous order (as k_part), where the launch asks for it: a wave's
+  // run of blocks ends inside a cache line that the next one's begins in
   const unsigned nb8 = gridDim.x & ~7u, b = blockIdx.x;
-  const unsigned block = b < nb8 ? (b & 7u) * (nb8 >> 3) + (b >> 3) : b;
+  const unsigned block = xcd && b < nb8 ? (b & 7u) * (nb8 >> 3) + (b >> 3) : b;
   blk2_tw_block<T, M, TRANS>(g, block, reinterpret_cast<T *>(smem_raw));
 }
 
@@ -1309,15 +1309,28 @@ hipError_t launch_m(const BlkArgs<T> &g, int lanes, hipStream_t st) {
   if constexpr (blk2tw_sizes(M)) {
     if (lanes == kTwistTiled) {
       const long long waves = (g.P + kWave / (2 * M) - 1) / (kWave / (2 * M));
-      // one-wave work-groups spread a small batch over all CUs and end
+      // One-wave work-groups spread a small batch over all CUs and end
       // together (N = 100, FP64, one / four waves: M = 4, P = 2500 69 / 82 us,
-      // M = 7, P = 5000 258 / 330; P = 16384, M = 5 435 / 423); the short
-      // blocks of M = 3 share more cache lines between waves (P = 5000 71 /
-      // 85, 8000 107 / 105)
-      const int wpb = waves < (M == 3 ? 640 : 2048) ? 1 : 4;
+      // M = 7, P = 5000 258 / 330; N = 128, M = 5, P = 8000, 1334 waves,
+      // 275 / 322, 12000, 2000 waves, 388 / 381, 16384 564 / 547; M = 7, P = 8000, 2000
+      // waves, 489 / 485).  The short blocks of M = 3 share more cache lines
+      // between waves, which four-wave groups use best just below one wave per
+      // SIMD, and from four waves per SIMD on (FP64, N = 128: P = 8000, 800 waves, 138 / 137 us; 12000 168 /
+      // 220; 16384 235 / 248; 32768, 3277 waves, 457 / 495; 49152 699 / 661).
+      const bool mid3 = sizeof(T) == 8 && waves >= 1024 && waves < 4096;
+      const int wpb = (M == 3 ? waves < 640 || mid3 : waves < 1792) ? 1 : 4;
+      // The XCD order shares a wave's cache lines with the next wave of its
+      // XCD while a row of the batch, about 32 waves * M elements of each
+      // matrix, stays in the L2s beside the rows on their way; past 6 MiB
+      // (FP64, N = 128, XCD / plain order: M = 4, P = 32768 635 / 643 us,
+      // 65536 1303 / 1278; M = 7, P = 8000 489 / 493, 49152 3032 / 2964; M =
+      // 8, P = 16384 1150 / 1127) the plain order keeps what is on its way
+      // closer together.  FP32 is equal or better in the XCD order throughout
+      // (M = 8, P = 65536 2358 / 2370).
+      const int xcd = sizeof(T) == 4 || 32 * waves * M * (long long)sizeof(T) < 6ll << 20;
       const size_t lds = blk2_tw_lds<T, M>() / 4 * wpb;
       hipLaunchKernelGGL((k_blk2_tw<T, M, TRANS>), dim3((unsigned)((waves + wpb - 1) / wpb)),
-                         dim3(wpb * kWave), lds, st, g);
+                         dim3(wpb * kWave), lds, st, g, xcd);
       return hipGetLastError();
     }
   }
