@@ -131,3 +131,39 @@ def test_other_streams_start_behind_torchs(on_host, monkeypatch, wait):
     autograd.trid_solve(*t, 0).sum().backward()
     start = ["wait"] * wait
     assert log == start + [("solve", wait)] + start + [("adjoint", wait)]
+
+
+class VadiLib:
+    """The variable-diffusivity entry points over host arrays."""
+
+    @staticmethod
+    def _grid(p, n):
+        return np.ctypeslib.as_array((C.c_double * n ** 3).from_address(p))
+
+    def tridVadiForward(self, kappa, u, nx, ny, nz, steps, lam, sync):
+        k, v = self._grid(kappa, nx), self._grid(u, nx)
+        v[:] = oracle.vadi_forward(k.copy(), v.copy(), nx, steps, lam)
+        return 0
+
+    def tridVadiLossGrad(self, kappa, u0, target, nx, ny, nz, steps, lam, ckpt, loss, gk, gu):
+        k, u, t = (self._grid(p, nx).copy() for p in (kappa, u0, target))
+        loss._obj.value, a, b = oracle.vadi_grad(k, u, t, nx, steps, lam)
+        self._grid(gk, nx)[:], self._grid(gu, nx)[:] = a, b
+        return 0
+
+
+@pytest.mark.parametrize("make", [_transposed, _sliced, _expanded])
+def test_vadi_grids_of_any_strides(monkeypatch, make):
+    """Grids that are not contiguous give what contiguous copies of them do."""
+    monkeypatch.setattr(autograd, "lib", VadiLib)
+    gen = torch.Generator().manual_seed(4)
+    grids = [make(torch.rand(5, 5, 5, generator=gen, dtype=torch.float64) + 0.5)
+             for _ in range(3)]
+    assert not any(t.is_contiguous() for t in grids)
+    kappa, u0, target = dense = [t.contiguous() for t in grids]
+    assert torch.equal(autograd.vadi_forward(*grids[:2], 2, 0.5),
+                       autograd.vadi_forward(kappa, u0, 2, 0.5))
+    got = autograd.vadi_loss_grad(*grids, 2, 0.5)
+    exp = autograd.vadi_loss_grad(*dense, 2, 0.5)
+    assert got[0] == exp[0]
+    assert torch.equal(got[1], exp[1]) and torch.equal(got[2], exp[2])

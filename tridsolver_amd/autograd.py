@@ -81,6 +81,7 @@ def _grid(t):
 
 def vadi_forward(kappa, u0, steps: int, lam: float):
     u = u0.clone().contiguous()
+    kappa = kappa.contiguous()  # the library takes dense grids
     nx, ny, nz = _grid(u)
     _check(lib().tridVadiForward(kappa.data_ptr(), u.data_ptr(), nx, ny, nz, int(steps),
                                  float(lam), 1), "tridVadiForward")
@@ -90,6 +91,7 @@ def vadi_forward(kappa, u0, steps: int, lam: float):
 def vadi_loss_grad(kappa, u0, target, steps: int, lam: float, ckpt: int = 4):
     """Returns (loss, grad_kappa, grad_u0)."""
     nx, ny, nz = _grid(u0)
+    kappa, u0, target = (t.contiguous() for t in (kappa, u0, target))
     gk = torch.empty_like(kappa)
     gu = torch.empty_like(u0)
     loss = C.c_double(0.0)
