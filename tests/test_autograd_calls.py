@@ -156,6 +156,7 @@ class VadiLib:
 def test_vadi_grids_of_any_strides(monkeypatch, make):
     """Grids that are not contiguous give what contiguous copies of them do."""
     monkeypatch.setattr(autograd, "lib", VadiLib)
+    monkeypatch.setattr(autograd, "_sync", lambda t: 0)
     gen = torch.Generator().manual_seed(4)
     grids = [make(torch.rand(5, 5, 5, generator=gen, dtype=torch.float64) + 0.5)
              for _ in range(3)]
@@ -167,3 +168,29 @@ def test_vadi_grids_of_any_strides(monkeypatch, make):
     exp = autograd.vadi_loss_grad(*dense, 2, 0.5)
     assert got[0] == exp[0]
     assert torch.equal(got[1], exp[1]) and torch.equal(got[2], exp[2])
+
+
+@pytest.mark.parametrize("wait", [0, 1])
+def test_vadi_starts_behind_torchs_stream(monkeypatch, wait):
+    """As for the solves: the copies of the grids are finished before a launch
+    on another stream than torch's."""
+    log = []
+
+    class Lib(VadiLib):
+        def tridVadiForward(self, *args):
+            log.append("forward")
+            return super().tridVadiForward(*args)
+
+        def tridVadiLossGrad(self, *args):
+            log.append("gradient")
+            return super().tridVadiLossGrad(*args)
+
+    monkeypatch.setattr(autograd, "lib", Lib)
+    monkeypatch.setattr(autograd, "_sync", lambda t: wait)
+    stream = SimpleNamespace(synchronize=lambda: log.append("wait"))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev=None: stream)
+    kappa, u0, target = (torch.ones(4, 4, 4, dtype=torch.float64) for _ in range(3))
+    autograd.vadi_forward(kappa, u0, 1, 0.5)
+    autograd.vadi_loss_grad(kappa, u0, target, 1, 0.5)
+    start = ["wait"] * wait
+    assert log == start + ["forward"] + start + ["gradient"]

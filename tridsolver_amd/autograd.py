@@ -83,6 +83,7 @@ def vadi_forward(kappa, u0, steps: int, lam: float):
     u = u0.clone().contiguous()
     kappa = kappa.contiguous()  # the library takes dense grids
     nx, ny, nz = _grid(u)
+    _ordered(u)
     _check(lib().tridVadiForward(kappa.data_ptr(), u.data_ptr(), nx, ny, nz, int(steps),
                                  float(lam), 1), "tridVadiForward")
     return u
@@ -95,6 +96,7 @@ def vadi_loss_grad(kappa, u0, target, steps: int, lam: float, ckpt: int = 4):
     gk = torch.empty_like(kappa)
     gu = torch.empty_like(u0)
     loss = C.c_double(0.0)
+    _ordered(u0)
     _check(lib().tridVadiLossGrad(kappa.data_ptr(), u0.data_ptr(), target.data_ptr(), nx, ny, nz,
                                   int(steps), float(lam), int(ckpt), C.byref(loss),
                                   gk.data_ptr(), gu.data_ptr()), "tridVadiLossGrad")
