@@ -22,20 +22,21 @@
  * past 64 chunks, one of two reduced solves: PCR through LDS, one barrier per
  * level, or PCR within each wave followed by a serial sweep across the
  * waves (three barriers).  Untuned, FP64 takes 5..8 rows up to 4096 rows with
- * PCR through LDS, FP32 the same unless a system has more than 4096 rows:
- * then 9..16 rows throughout with the per-wave reduced solve.  With the autotuner on (tridSetAutotune(1)
- * when the plan is created) the plan times whole solves of a synthetic batch
- * with its own lengths (a uniform sample of the systems past 2^27 unknowns),
- * in buffers of its own, and from the untuned choices changes one class at a
- * time, from the most to the fewest unknowns, keeping a change that makes
- * the whole solve faster by more than 2 %.
+ * PCR through LDS, FP32 the same unless a system has 4097..8192 rows: then
+ * 9..16 rows throughout with the per-wave reduced solve (longer systems are
+ * solved apart and change nothing here).  With the autotuner on
+ * (tridSetAutotune(1) when the plan is created) the plan times whole solves of
+ * a synthetic batch with its own lengths (a uniform sample of the systems past
+ * 2^27 unknowns), in buffers of its own, and from the untuned choices changes
+ * one class at a time, from the most to the fewest unknowns, keeping a change
+ * that makes the whole solve faster by more than 2 %.
  * The plan builds a work list per family ordered from the most to the least
  * expensive item; each solve is one launch of a persistent kernel per
  * family present, whose work-groups take every grid-th item.  Systems
- * longer than 8192 rows are solved after it: the longest of them one by one, each as a strided batch of one
- * system (tridXmtsvStridedBatch, split-line solve past 8192 rows), the rest
- * by a one-thread-per-system launch; the plan picks the split by a cost
- * model (untuned: a one-system solve ~25 us, the one-thread launch ~0.5 us
+ * longer than 8192 rows are solved after it: the longest of them one by one,
+ * each as a strided batch of one system (tridXmtsvStridedBatch, split-line
+ * solve past 8192 rows), the rest by a one-thread-per-system launch; the plan
+ * picks the split by a cost model (untuned: a one-system solve ~25 us, the one-thread launch ~0.5 us
  * per row of its longest system; the autotuner measures both on the plan's
  * longest system).
  * A plan may be used for any arrays with the same offsets; a solve changes

@@ -298,9 +298,9 @@ __device__ __forceinline__ void rag_dispatch(const RagArgs<T> &g, const RagItem 
 // is sorted by cost and items of one bin cost the same, so the shares come out
 // even without a work queue.  (One device-wide counter for the next item and
 // the finished work-groups serialised 512 groups on one address: 50000 FP64
-// systems of 4..64, 8..512 and 8..4096 rows took 71, 110 and 333 us, now 37,
-// 70 and 304; one work-group per item 36, 74 and 291.)  RLO..RHI: the chunk
-// lengths of the launch's items.
+// systems of 4..64, 8..512 and 8..4096 rows, lengths log-uniform, took 74, 111
+// and 320 us, now 38, 72 and 282; one work-group per item 38, 75 and 284.)
+// RLO..RHI: the chunk lengths of the launch's items.
 template <typename T, int RLO, int RHI>
 __global__ void __launch_bounds__(kRagThreads) k_ragged(RagArgs<T> g) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -445,15 +445,15 @@ bool red_matters(int c, int f) {
   return bin_of(Lmax, f, R) > 6;
 }
 
-// past_f0: the batch has systems of more than 4096 rows
+// past_f0: the batch has systems of 4097..8192 rows
 RagChoice default_choice(int c, bool dbl, bool past_f0) {
-  // measured on MI355X, us for families 0 / 1.  FP64: family 0 up to 4096
-  // rows, family 1 past it, PCR through LDS (50000 systems of 8..4096 rows
-  // 305 / 343, of 8..512 71 / 94; 24000 of 8..6000 rows 216, 224 all in
-  // family 1).  FP32: family 0 and PCR through LDS (50000 of 8..512 rows 43 /
-  // 56, 12000 of 8..4096 rows 44 / 49), unless the batch needs family 1
-  // anyway: then all of it, in one launch, with the per-wave reduced solve
-  // (24000 of 8..6000 rows 116 in two launches, 109)
+  // measured on MI355X, us for families 0 / 1, lengths log-uniform.  FP64:
+  // family 0 up to 4096 rows, family 1 past it, PCR through LDS (50000 systems
+  // of 8..4096 rows 283 / 343, of 8..512 71 / 96; 24000 of 8..6000 rows 218,
+  // 226 all in family 1).  FP32: family 0 and PCR through LDS (50000 of 8..512
+  // rows 44 / 57, 12000 of 8..4096 rows 44 / 49), unless the batch needs family
+  // 1 anyway: then all of it, in one launch, with the per-wave reduced solve
+  // (24000 of 8..6000 rows 117 in two launches, 110; 50000 224, 222)
   RagChoice ch;
   ch.fam = c < 10 && (dbl || !past_f0) ? 0 : 1;
   ch.red = dbl || !past_f0 ? 0 : 1;
