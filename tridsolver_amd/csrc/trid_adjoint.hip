@@ -249,9 +249,22 @@ namespace {
 // 173 and 178 us for forward and backward through autograd).  kind 0 where
 // the staging does not apply: arrays not 16-byte aligned, or padded systems
 // that share a wave.
-PartCfg adj_rows(int N, bool aligned, bool dense) {
+// Batches of at most one wave of 8-row chunks per SIMD (65536 lanes) wait on
+// each chunk's serial rows, not on bandwidth: the shortest chunks, in one-wave
+// work-groups (FP64, N x systems, against the fewest rows in 256 threads: 20 x
+// 1000 10.7 -> 7.9 us, 40 x 40 9.9 -> 7.9, 1000 x 10 11.4 -> 10.2, 90 x 4000
+// 13.5 -> 11.6; above the line 600 x 800 14.7 -> 15.7, 150 x 8000 17.8 -> 20.3).
+// Past 256 chunks per system the reduced solve costs more than the rows save
+// (3000 x 5, 512 chunks of 8 rows 14.6 us, 256 of 12 13.4).
+PartCfg adj_rows(int N, long long nsys, bool aligned, bool dense) {
   PartCfg best;
   best.kind = 0;
+  const PartCfg small = make_cfg(0, 8, N, 0, kWave);
+  if (N <= 2048 && gstage_ok(small, aligned, dense) && nsys << small.cps_log2 <= 65536) {
+    best = small;
+    best.vec = 4;
+    return best;
+  }
   for (int R : {8, 12, 16}) {
     PartCfg c = make_cfg(0, R, N, 0, 256);
     if (!gstage_ok(c, aligned, dense)) continue;
@@ -314,7 +327,7 @@ tridStatus_t strided_adjoint(const T *a, const T *b, const T *c, const T *x, con
     const PartCfg w = strided_wide(D.N, D.nsys, sizeof(T), rr);
     if (w.kind == 1) cfg = w;
   } else {
-    const PartCfg s = adj_rows(D.N, aligned, dense);
+    const PartCfg s = adj_rows(D.N, D.nsys, aligned, dense);
     if (s.kind == 1) cfg = s;
   }
   const size_t bytes = (size_t)ext * sizeof(T);
