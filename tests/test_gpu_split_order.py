@@ -51,3 +51,30 @@ def test_policy_of_whole_lines(w, k, tags):
     band = np.array([[0.0] + [-1.0] * (k - 1), [4.0] * k, [-1.0] * (k - 1) + [0.0]])
     x = torch.from_numpy(solve_banded((1, 1), band, np.ones(k))).cuda()[:, None]
     assert (d - x).abs().max().item() <= 1e-14
+
+
+@pytest.mark.parametrize("segments,fits", [(15800, True), (16200, True), (16400, False)])
+def test_fixed_scratch_limit(segments, fits):
+    """FP64, 64 systems of 64-row segments whose reduced systems are split
+    again: in the systems' order the scratch is 4224 bytes per segment (4 arrays
+    of 2 rows for each system's segment, and of 2 rows per 32 of them), as
+    contiguous systems 4112.  A solve is refused where neither fits 64 MiB."""
+    import ctypes as C
+
+    import torch
+    w, k = 64, segments * 64
+    gen = torch.Generator(device="cuda").manual_seed(segments)
+    x, a, c = (torch.rand((k, w), generator=gen, dtype=torch.float64, device="cuda")
+               for _ in range(3))
+    b = a + c + 1.5
+    d = b * x
+    d[1:] -= a[1:] * x[:-1]
+    d[:-1] -= c[:-1] * x[1:]
+    a.neg_(), c.neg_()
+    dims = (C.c_int * 2)(w, k)
+    got = d.clone()
+    st = ta.lib().tridDmtsvStridedBatchNoAlloc(*(t.data_ptr() for t in (a, b, c, got)), None, 2,
+                                               1, dims, dims, None, 1)
+    assert st == (0 if fits else 3), ta.last_error()
+    want = x if fits else d
+    assert ((got - want).abs().max() / want.abs().max()).item() <= (1e-12 if fits else 0.0)

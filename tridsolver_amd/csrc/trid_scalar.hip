@@ -203,29 +203,30 @@ SysDesc reduced_desc(int order, int P, long long ns) {
 // long systems' order, whose lanes read and write whole lines where contiguous
 // ones scatter 2P apart (4096 x 8192 rows FP64 402 against 414 us, 333 x 4096
 // x 30 638 against 701); so do nested segments (64 x 2^19 rows 427 against
-// 464).
+// 464), whose shorter segments take some 3 % more workspace: `contig` keeps all
+// of them contiguous.
 template <typename T>
-int reduced_order(int order, int P, long long ns) {
-  if (order == 0) return 0;
+int reduced_order(int order, int P, long long ns, bool contig) {
+  if (order == 0 || contig) return 0;
   return ns < 1024 && reduced_cfg<T>(0, reduced_desc(0, P, ns)).kind == 1 ? 0 : 1;
 }
 
 // Workspace (elements) of a split-line solve, including its recursive
 // reduced solves.
 template <typename T>
-long long split_ws_elems(const PartCfg &cfg, int N, long long nsys) {
+long long split_ws_elems(const PartCfg &cfg, int N, long long nsys, bool contig = false) {
   const long long L = (long long)cfg.R << cfg.cps_log2;
   const long long P = (N + L - 1) / L;
   long long need = 4 * round4(2 * P * nsys);
-  const int ro = reduced_order<T>(cfg.order, (int)P, nsys);
+  const int ro = reduced_order<T>(cfg.order, (int)P, nsys, contig);
   const PartCfg cr = reduced_cfg<T>(ro, reduced_desc(ro, (int)P, nsys));
-  if (cr.kind != 1) need += split_ws_elems<T>(cr, (int)(2 * P), nsys);
+  if (cr.kind != 1) need += split_ws_elems<T>(cr, (int)(2 * P), nsys, contig);
   return need;
 }
 
 template <typename T, int INC>
 hipError_t split_solve(const PartCfg &cfg, const T *a, const T *b, const T *c, T *d,
-                       T *u, const SysDesc &D, hipStream_t st, T *ws) {
+                       T *u, const SysDesc &D, hipStream_t st, T *ws, bool contig = false) {
   const int order = cfg.order;
   const int L = cfg.R << cfg.cps_log2;
   const int N = D.N, P = (N + L - 1) / L;
@@ -240,7 +241,7 @@ hipError_t split_solve(const PartCfg &cfg, const T *a, const T *b, const T *c, T
   so.nsys = ns;
   so.P = P;
   so.N = N;
-  const int ro = reduced_order<T>(order, P, ns);
+  const int ro = reduced_order<T>(order, P, ns, contig);
   so.rs_row = ro == 0 ? 1 : ns;
   so.rs_sys = ro == 0 ? 2LL * P : 1;
 
@@ -278,7 +279,8 @@ hipError_t split_solve(const PartCfg &cfg, const T *a, const T *b, const T *c, T
   if (cr.kind == 1)
     e = launch_part<T, 0>(cr, CoefArrays<T>{so.ra, so.rb, so.rc}, so.rd, nullptr, Dr, st);
   else
-    e = split_solve<T, 0>(cr, so.ra, so.rb, so.rc, so.rd, nullptr, Dr, st, ws + 4 * n2);
+    e = split_solve<T, 0>(cr, so.ra, so.rb, so.rc, so.rd, nullptr, Dr, st, ws + 4 * n2,
+                          contig);
   if (e != hipSuccess) return e;
 
   // 3. independent segments, couplings from the reduced solution
@@ -311,9 +313,11 @@ tridStatus_t run_cfg(const PartCfg &cfg, const T *a, const T *b, const T *c,
                      size_t fixed_bytes = 0) {
   hipError_t e;
   if (cfg.kind == 2 || cfg.kind == 4) {
-    const size_t bytes =
-        cfg.kind == 2 ? 2 * (size_t)D.N * (size_t)D.nsys * sizeof(T)
-                      : (size_t)split_ws_elems<T>(cfg, D.N, D.nsys) * sizeof(T);
+    size_t bytes = cfg.kind == 2 ? 2 * (size_t)D.N * (size_t)D.nsys * sizeof(T)
+                                 : (size_t)split_ws_elems<T>(cfg, D.N, D.nsys) * sizeof(T);
+    // fixed scratch that the faster order does not fit takes the smaller one
+    const bool contig = cfg.kind == 4 && fixed && bytes > fixed_bytes;
+    if (contig) bytes = (size_t)split_ws_elems<T>(cfg, D.N, D.nsys, true) * sizeof(T);
     T *ws;
     if (fixed) {
       if (bytes > fixed_bytes)
@@ -328,7 +332,7 @@ tridStatus_t run_cfg(const PartCfg &cfg, const T *a, const T *b, const T *c,
     if (cfg.kind == 2)
       e = launch_fallback<T, INC>(a, b, c, d, u, D, st, ws);
     else
-      e = split_solve<T, INC>(cfg, a, b, c, d, u, D, st, ws);
+      e = split_solve<T, INC>(cfg, a, b, c, d, u, D, st, ws, contig);
   } else {
     e = launch_part<T, INC>(cfg, CoefArrays<T>{a, b, c}, d, u, D, st);
   }
