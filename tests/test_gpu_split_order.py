@@ -76,5 +76,10 @@ def test_fixed_scratch_limit(segments, fits):
     st = ta.lib().tridDmtsvStridedBatchNoAlloc(*(t.data_ptr() for t in (a, b, c, got)), None, 2,
                                                1, dims, dims, None, 1)
     assert st == (0 if fits else 3), ta.last_error()
+    if fits:  # the allocating form gives the same bits
+        other = d.clone()
+        assert ta.lib().tridDmtsvStridedBatch(*(t.data_ptr() for t in (a, b, c, other)), None, 2,
+                                              1, dims, dims, None, 1) == 0
+        assert torch.equal(got, other)
     want = x if fits else d
     assert ((got - want).abs().max() / want.abs().max()).item() <= (1e-12 if fits else 0.0)

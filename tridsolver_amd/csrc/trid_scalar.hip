@@ -315,9 +315,14 @@ tridStatus_t run_cfg(const PartCfg &cfg, const T *a, const T *b, const T *c,
   if (cfg.kind == 2 || cfg.kind == 4) {
     size_t bytes = cfg.kind == 2 ? 2 * (size_t)D.N * (size_t)D.nsys * sizeof(T)
                                  : (size_t)split_ws_elems<T>(cfg, D.N, D.nsys) * sizeof(T);
-    // fixed scratch that the faster order does not fit takes the smaller one
-    const bool contig = cfg.kind == 4 && fixed && bytes > fixed_bytes;
-    if (contig) bytes = (size_t)split_ws_elems<T>(cfg, D.N, D.nsys, true) * sizeof(T);
+    // Where only the smaller order fits the no-allocation form's scratch, both
+    // forms take it and give the same bits
+    bool contig = false;
+    if (cfg.kind == 4 && bytes > TRID_NOALLOC_SCRATCH_BYTES) {
+      const size_t least = (size_t)split_ws_elems<T>(cfg, D.N, D.nsys, true) * sizeof(T);
+      contig = least <= TRID_NOALLOC_SCRATCH_BYTES;
+      if (contig) bytes = least;
+    }
     T *ws;
     if (fixed) {
       if (bytes > fixed_bytes)
@@ -596,8 +601,10 @@ tridStatus_t solve(const T *a, const int *a_pads, const T *b,
   // a line for their chunk's next rows read it again when it streams
   // ([200, 180, 250] FP64 Inc with lines padded to 208, 357 MiB: 88 / 105 us;
   // over 270..380 MiB 1.13 to 1.28 times, scalar rows 1.46 to 1.66 times).
-  // Strided rows keep cached up to the rule's 384 MiB: [180, 200, 250] FP64,
-  // 275 MiB, solvedim 1: 64 / 78 and 78 / 78
+  // Strided rows keep cached up to the rule's 384 MiB: cached / mixed, the
+  // same arrays again, two sets and four in turn: [180, 200, 250] FP64, 275
+  // MiB, solvedim 1: 63 / 79, 79 / 78 and 79 / 87; [200, 180, 250] FP64 Inc,
+  // 357 MiB, solvedim 2: 100 / 86, 107 / 95 and 107 / 112
   const bool whole_loads = cfg.vec >= 2 || (cfg.vec == 1 && cfg.R * sizeof(T) == 16);
   if (!tuned && order == 0 && cfg.kind == 1 && cfg.cp == kCached && footprint > kMallBytes &&
       whole_loads)
