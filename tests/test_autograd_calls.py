@@ -133,6 +133,20 @@ def test_other_streams_start_behind_torchs(on_host, monkeypatch, wait):
     assert log == start + [("solve", wait)] + start + [("adjoint", wait)]
 
 
+def test_saved_tensor_hooks_of_any_strides(on_host):
+    """Hooks that give the saved tensors back with other strides change nothing."""
+    dims, shape = [6, 5, 4], (4, 5, 6)
+    t = [torch.from_numpy(v).reshape(shape) for v in dd_system(dims, 1, np.float64, seed=3)]
+    g = torch.from_numpy(np.random.default_rng(2).uniform(-1, 1, shape))
+    grads = []
+    for unpack in (lambda v: v, _transposed):
+        leaves = [v.clone().requires_grad_(True) for v in t]
+        with torch.autograd.graph.saved_tensors_hooks(lambda v: v, unpack):
+            x = autograd.trid_solve(*leaves, 1)
+        grads.append(torch.autograd.grad(x, leaves, g))
+    assert all(torch.equal(u, v) for u, v in zip(*grads))
+
+
 class VadiLib:
     """The variable-diffusivity entry points over host arrays."""
 

@@ -57,7 +57,7 @@ class TridSolve(torch.autograd.Function):
         # the adjoint takes dense arrays; the copies, like gx's, are dropped on
         # torch's stream, behind the launch that reads them
         a, b, c, x = ctx.saved_tensors
-        a, b, c = a.contiguous(), b.contiguous(), c.contiguous()
+        a, b, c, x = a.contiguous(), b.contiguous(), c.contiguous(), x.contiguous()
         gx = gx.contiguous()
         ga, gb, gc, gd = (torch.empty_like(x) for _ in range(4))
         dims = dims_of(x)
