@@ -94,7 +94,7 @@ def vadi_forward(kappa, u0, steps: int, lam: float):
 def vadi_loss_grad(kappa, u0, target, steps: int, lam: float, ckpt: int = 4):
     """Returns (loss, grad_kappa, grad_u0)."""
     nx, ny, nz = _grid(u0)
-    kappa, u0, target = (t.contiguous() for t in (kappa, u0, target))
+    kappa, u0, target = kappa.contiguous(), u0.contiguous(), target.contiguous()
     gk = torch.empty_like(kappa)
     gu = torch.empty_like(u0)
     loss = C.c_double(0.0)
